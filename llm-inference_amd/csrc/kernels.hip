@@ -2349,49 +2349,283 @@ extern "C" void attention_forward_noalloc(bf16 *out, const bf16 *q, const bf16 *
 // temperature sampling (src/kernels.cu:546-597)
 // ------------------------------------------------------------------------------------------
 
-// Inverse-CDF sampling from softmax(x * inv_temp), one workgroup of SAMPLE_T threads. The
-// additions keep the reference's order, so the chosen index follows from the weights alone: the
-// row's max; thread t adds the weights exp((x - max) * inv_temp) of the contiguous chunk
-// [t c, t c + c) in order (c = ceil(n / SAMPLE_T)); thread 0 adds the chunk sums in order for the
-// total, walks them to the chunk holding u * total (never past the last) and then that chunk's
-// elements to the first whose running sum passes it (-1 if none does). Not on the decode path.
+// Inverse-CDF sampling from softmax(x * inv_temp). The additions keep the reference's order, so the
+// chosen index follows from the weights alone: the row's max; chunk k of SAMPLE_T contiguous chunks
+// [k c, k c + c) adds its weights exp((x - max) * inv_temp) in order (c = ceil(n / SAMPLE_T)); the
+// chunk sums are added in order for the total and walked to the chunk holding u * total (never past
+// the last), then that chunk's elements to the first whose running sum passes it (-1 if none does).
+//
+// Two launches for long rows: sample_kernel, one workgroup, takes the max (a row of 151936 is 300 KB,
+// read from L2); sample_sums_kernel spreads the weights, which are most of the work, over SAMPLE_WGS
+// workgroups, and the last of them to finish adds the chunk sums and draws. Between the two the max
+// and the chunk sums live in one of SAMPLE_SLOTS library-owned slots, taken by the first launch with
+// an atomic exchange and given back by the second, so calls on any streams may overlap; `out` itself
+// carries the slot (as -2 - slot) from one launch to the next. With every slot taken the first
+// launch draws alone, as it does for rows of up to SAMPLE_ALONE.
+//
+// Bound by its serial chains, which the order of the additions fixes: 1024 dependent adds for the
+// total (5.5 us measured), about 150 per chunk; the rest is two launches and four round trips to
+// memory. 151936 logits: 119.2 us on one workgroup that also computed every weight, 19.6 us now
+// (6.0 + 13.6); one launch alone now 72 us. The line at SAMPLE_ALONE: alone 9.7 / 11.4 / 16.3 / 22.6
+// us at 4096 / 8192 / 16384 / 32768 logits, spread 15.0-15.5 us at each.
 constexpr int SAMPLE_T = 1024;
+constexpr int SAMPLE_WGS = 64, SAMPLE_ROWS = SAMPLE_T / SAMPLE_WGS;  // chunks per workgroup
+constexpr int SAMPLE_PIECE = 256;  // weights of a chunk staged at a time
+constexpr int SAMPLE_SLOTS = 16;
+constexpr int SAMPLE_ALONE = 12288;  // longest row drawn in one launch
 
+struct SampleSlot {
+    unsigned busy;   // taken by a call
+    unsigned done;   // workgroups of the second launch that have published their sums
+    float max;
+    float pad[29];
+    float sums[SAMPLE_T];
+};
+static __device__ SampleSlot g_sample_slots[SAMPLE_SLOTS];
+
+// 16 consecutive floats of LDS (16-byte aligned), all requested at once.
+__device__ __forceinline__ void ld_lds16(const float *p, float (&v)[16]) {
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    const f32x4 *q = (const f32x4 *)p;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const f32x4 a = q[i];
+        v[4 * i] = a.x;
+        v[4 * i + 1] = a.y;
+        v[4 * i + 2] = a.z;
+        v[4 * i + 3] = a.w;
+    }
+}
+
+__device__ __forceinline__ void st_lds16(float *p, const float (&v)[16]) {
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    f32x4 *q = (f32x4 *)p;
+#pragma unroll
+    for (int i = 0; i < 4; i++) q[i] = f32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+}
+
+// The draw from the SAMPLE_T chunk sums in LDS, by the whole workgroup (every thread calls it after
+// a barrier). Prefix sums of non-negative weights never decrease, so the walk over the chunks is
+// done on the ends of 64 segments of 16 chunks first (lane s keeps the running sum after segment s:
+// the additions of the total itself), then inside one segment. One wave runs each serial chain.
+__device__ __forceinline__ void sample_draw(int *out, const bf16 *x, int n, float inv_temp, float u,
+                                            float mx, const float *sums, float *piece, float *share) {
+    const int t = threadIdx.x, lane = t & 63;
+    const int chunk = (n + SAMPLE_T - 1) / SAMPLE_T;
+    if (t < 64) {
+        // segments that hold chunks with elements (the sums past them are zeros, which add nothing)
+        const int segs = ((n + chunk - 1) / chunk + 15) / 16;
+        float total = 0.0f, end = 0.0f, v[16], w[16];
+        ld_lds16(sums, v);
+        for (int s = 0; s < segs; s += 2) {  // two segments a step, each read while the other is added
+            ld_lds16(sums + 16 * min(s + 1, 63), w);
+#pragma unroll
+            for (int j = 0; j < 16; j++) total += v[j];
+            end = lane >= s ? total : end;
+            ld_lds16(sums + 16 * min(s + 2, 63), v);
+            if (s + 1 < segs) {
+#pragma unroll
+                for (int j = 0; j < 16; j++) total += w[j];
+            }
+            end = lane > s ? total : end;
+        }
+        const float target = u * total;
+        const unsigned long long past = __ballot(!(end <= target));
+        const int s = past ? __ffsll(past) - 1 : 63;
+        float cdf = s > 0 ? __shfl(end, s - 1) : 0.0f;
+        int k = 16 * s;
+        while (k < SAMPLE_T - 1 && cdf + sums[k] <= target) cdf += sums[k++];
+        if (t == 0) {
+            share[0] = cdf;
+            share[1] = target;
+            share[2] = __int_as_float(k);
+        }
+    }
+    __syncthreads();
+    const float cdf = share[0], target = share[1];
+    const int k = __float_as_int(share[2]);
+    const long long start = (long long)k * chunk;
+    const int count = start >= n ? 0 : (int)(n - start < chunk ? n - start : chunk);
+    int chosen = -1;
+    float run = 0.0f;
+    for (int b = 0; b < count; b += SAMPLE_PIECE) {
+        const int len = min(SAMPLE_PIECE, count - b);
+        if (t < SAMPLE_PIECE)
+            piece[t] = t < len ? exp_f32((bf2f(x[start + b + t]) - mx) * inv_temp) : 0.0f;
+        __syncthreads();
+        if (t < 64 && chosen < 0) {
+            // the running sums in place (past the end they add zeros), then the first that passes
+            for (int j = 0; j < len; j += 16) {
+                float v[16];
+                ld_lds16(piece + j, v);
+#pragma unroll
+                for (int i = 0; i < 16; i++) v[i] = run = run + v[i];
+                st_lds16(piece + j, v);
+            }
+            for (int j = 0; j < len && chosen < 0; j += 64) {
+                const unsigned long long hit =
+                    __ballot(j + lane < len && cdf + piece[min(j + lane, len - 1)] > target);
+                if (hit) chosen = (int)(start + b + j) + __ffsll(hit) - 1;
+            }
+        }
+        __syncthreads();
+    }
+    if (t == 0) *out = chosen;
+}
+
+// The max of the row, then either the slot for sample_sums_kernel (spread != 0) or the whole draw.
+// vec: x is 16-byte aligned.
 __global__ __launch_bounds__(SAMPLE_T) void sample_kernel(int *out, const bf16 *x, int n,
-                                                          float inv_temp, float u) {
-    __shared__ float sums[SAMPLE_T];
+                                                          float inv_temp, float u, int vec,
+                                                          int spread) {
+    __shared__ __align__(16) float sums[SAMPLE_T];
+    __shared__ __align__(16) float piece[SAMPLE_PIECE];
     __shared__ float wmax[SAMPLE_T / 64];
+    __shared__ float share[3];
+    __shared__ int s_slot;
     const int t = threadIdx.x;
     float m = -__builtin_huge_valf();
-    for (int i = t; i < n; i += SAMPLE_T) m = fmaxf(m, bf2f(x[i]));
+    int done = 0;
+    if (vec) {
+        constexpr int U = 8;  // 16-byte loads of a thread in flight (past the end: the last chunk again)
+        const int n_chunks = n / 8;
+        for (int c0 = 0; c0 < n_chunks; c0 += U * SAMPLE_T) {
+            u32x4 v[U];
+#pragma unroll
+            for (int i = 0; i < U; i++)
+                v[i] = ld16(x + 8 * (size_t)min(c0 + i * SAMPLE_T + t, n_chunks - 1));
+#pragma unroll
+            for (int i = 0; i < U; i++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) m = fmaxf(m, elem(v[i], e));
+        }
+        done = n_chunks * 8;
+    }
+    for (int i = done + t; i < n; i += SAMPLE_T) m = fmaxf(m, bf2f(x[i]));
     m = wave_max(m);
     if ((t & 63) == 0) wmax[t >> 6] = m;
     __syncthreads();
     float mx = wmax[0];
+#pragma unroll
     for (int w = 1; w < SAMPLE_T / 64; w++) mx = fmaxf(mx, wmax[w]);  // max: any order
+    if (spread) {
+        if (t < 64) {
+            // lanes 0 .. SAMPLE_SLOTS - 1 look at one slot each, the lowest free one is taken
+            int slot = -1;
+            bool free = t < SAMPLE_SLOTS &&
+                        __hip_atomic_load(gptr(&g_sample_slots[t & (SAMPLE_SLOTS - 1)].busy),
+                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
+            unsigned long long left = __ballot(free);
+            while (left && slot < 0) {
+                const int s = __ffsll(left) - 1;
+                left &= left - 1;
+                unsigned was = 1;
+                if (t == 0)
+                    was = __hip_atomic_exchange(gptr(&g_sample_slots[s].busy), 1u, __ATOMIC_ACQUIRE,
+                                                __HIP_MEMORY_SCOPE_AGENT);
+                if (__builtin_amdgcn_readfirstlane(was) == 0) slot = s;
+            }
+            if (t == 0) {
+                s_slot = slot;
+                if (slot >= 0) {
+                    __hip_atomic_store(gptr(&g_sample_slots[slot].max), mx, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_store(gptr(&g_sample_slots[slot].done), 0u, __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+                    *out = -2 - slot;
+                }
+            }
+        }
+        __syncthreads();
+        if (s_slot >= 0) return;
+    }
     const int chunk = (n + SAMPLE_T - 1) / SAMPLE_T;
-    const int start = t * chunk, end = min(start + chunk, n);
+    const long long start = (long long)t * chunk, end = min(start + chunk, (long long)n);
     float acc = 0.0f;
-    for (int i = start; i < end; i++) acc += exp_f32((bf2f(x[i]) - mx) * inv_temp);
+    for (long long i = start; i < end; i++) acc += exp_f32((bf2f(x[i]) - mx) * inv_temp);
     sums[t] = acc;
     __syncthreads();
-    if (t != 0) return;
-    float total = 0.0f;
-    for (int k = 0; k < SAMPLE_T; k++) total += sums[k];
-    const float target = u * total;
-    float cdf = 0.0f;
-    int k = 0;
-    while (k < SAMPLE_T - 1 && cdf + sums[k] <= target) cdf += sums[k++];
-    int chosen = -1;
-    float run = 0.0f;
-    for (int i = k * chunk; i < min(k * chunk + chunk, n); i++) {
-        run += exp_f32((bf2f(x[i]) - mx) * inv_temp);
-        if (cdf + run > target) {
-            chosen = i;
-            break;
+    sample_draw(out, x, n, inv_temp, u, mx, sums, piece, share);
+}
+
+// Workgroup w: the sums of chunks [w SAMPLE_ROWS, (w + 1) SAMPLE_ROWS). All threads compute the
+// weights of a piece of each chunk into LDS (four chunks per wave, one lane per weight), then lane r
+// of the first wave adds chunk r's in order. The workgroup that publishes last draws.
+__global__ __launch_bounds__(256) void sample_sums_kernel(int *out, const bf16 *x, int n,
+                                                          float inv_temp, float u) {
+    constexpr int R = SAMPLE_ROWS, P = SAMPLE_PIECE, RW = R / 4;
+    __shared__ __align__(16) float stage[R * (P + 1)];  // padded rows: lanes 0..R-1 read one column
+    __shared__ float share[3];
+    __shared__ int s_last;
+    static_assert(R * (P + 1) >= SAMPLE_T + P, "the draw reuses the staging");
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    const int chunk = (n + SAMPLE_T - 1) / SAMPLE_T;
+    const int k0 = blockIdx.x * R;
+    // this lane's elements of the piece at b, clamped into the row (those past a chunk's end or the
+    // row's are not added)
+    uint16_t v[RW][P / 64];
+    const auto request = [&](int b) {
+#pragma unroll
+        for (int r = 0; r < RW; r++)
+#pragma unroll
+            for (int j = 0; j < P / 64; j++) {
+                const long long at = (long long)(k0 + w * RW + r) * chunk + b + lane + 64 * j;
+                v[r][j] = x[min(at, (long long)n - 1)];
+            }
+    };
+    request(0);  // before the slot's two dependent reads
+    const int slot = -2 - *out;
+    if (slot < 0 || slot >= SAMPLE_SLOTS) return;  // the first launch has drawn (or *out is no slot)
+    SampleSlot &sl = g_sample_slots[slot];
+    const float mx = __hip_atomic_load(gptr(&sl.max), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    float acc = 0.0f;
+    for (int b = 0; b < chunk; b += P) {
+        const int len = min(P, chunk - b);
+#pragma unroll
+        for (int r = 0; r < RW; r++)
+#pragma unroll
+            for (int j = 0; j < P / 64; j++)
+                if (64 * j < len)
+                    stage[(w * RW + r) * (P + 1) + lane + 64 * j] =
+                        exp_f32((bf2f(v[r][j]) - mx) * inv_temp);
+        if (b + P < chunk) request(b + P);
+        __syncthreads();
+        if (t < R) {
+            // chunk k0 + t's weights of the piece that exist, in order, 16 LDS reads in flight
+            const long long at = (long long)(k0 + t) * chunk + b;
+            const int have = at >= n ? 0 : (int)min((long long)len, n - at);
+            const float *row = stage + t * (P + 1);
+            int j = 0;
+            for (; j + 16 <= have; j += 16) {
+                float e[16];
+#pragma unroll
+                for (int i = 0; i < 16; i++) e[i] = row[j + i];
+#pragma unroll
+                for (int i = 0; i < 16; i++) acc += e[i];
+            }
+            for (; j < have; j++) acc += row[j];
         }
+        __syncthreads();
     }
-    *out = chosen;
+    if (t < R)
+        __hip_atomic_store(gptr(&sl.sums[k0 + t]), acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (t == 0)  // the same wave's stores come before its arrival
+        s_last = __hip_atomic_fetch_add(gptr(&sl.done), 1u, __ATOMIC_ACQ_REL,
+                                        __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+    __syncthreads();
+    if (!s_last) return;
+    float *sums = stage, *piece = stage + SAMPLE_T;
+    float got[SAMPLE_T / 256];
+#pragma unroll
+    for (int i = 0; i < SAMPLE_T / 256; i++)
+        got[i] = __hip_atomic_load(gptr(&sl.sums[t + 256 * i]), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int i = 0; i < SAMPLE_T / 256; i++) sums[t + 256 * i] = got[i];
+    __syncthreads();
+    if (t == 0)  // nothing reads the slot any more
+        __hip_atomic_store(gptr(&sl.busy), 0u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    sample_draw(out, x, n, inv_temp, u, mx, sums, piece, share);
 }
 
 extern "C" void sample_forward(int *out, const bf16 *x, int n, float inv_temp, float u,
@@ -2400,7 +2634,10 @@ extern "C" void sample_forward(int *out, const bf16 *x, int n, float inv_temp, f
         llm_fail("sample: n %d must be positive", n);
         return;
     }
-    sample_kernel<<<1, SAMPLE_T, 0, stream>>>(out, x, n, inv_temp, u);
+    const int spread = n > SAMPLE_ALONE;
+    sample_kernel<<<1, SAMPLE_T, 0, stream>>>(out, x, n, inv_temp, u, aligned16(x) ? 1 : 0, spread);
+    if (!LAUNCH_OK() || !spread) return;
+    sample_sums_kernel<<<SAMPLE_WGS, 256, 0, stream>>>(out, x, n, inv_temp, u);
     LAUNCH_OK();
 }
 

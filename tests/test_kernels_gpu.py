@@ -668,6 +668,57 @@ def test_sample_forward(gpu, oracle):
                 assert int(out.item()) == oracle.sample(row, inv_temp, u), (row.size, inv_temp, u)
 
 
+# chunk lengths around the staged piece (256 weights), rows around the one-launch limit (12288)
+@pytest.mark.parametrize("n", [1, 16, 1025, 12288, 12289, 16 * 1024 + 1, 262144, 262145, 300001])
+def test_sample_forward_row_lengths(gpu, oracle, n):
+    """Both forms of the draw (one launch; sums spread over workgroups, drawn by the last) equal the
+    oracle: random rows, a row that is mostly -inf, rows with a NaN and an inf, an unaligned view."""
+    import torch
+    ident(f"sample_forward row of {n}")
+    rng = np.random.default_rng(n)
+    out = torch.zeros(1, dtype=torch.int32, device="cuda")
+    sparse = np.full(n, 0xFF80, np.uint16)  # -inf
+    sparse[rng.integers(0, n, 5)] = rand_bf16(rng, 5)
+    nan, inf = rand_bf16(rng, n), rand_bf16(rng, n)
+    nan[n // 2], inf[n // 3] = 0x7FC0, 0x7F80
+    for row in (rand_bf16(rng, n, 2.0), sparse, nan, inf):
+        xd = dev(np.concatenate([row[:1], row]))
+        for x in (dev(row), xd[1:]):
+            for inv_temp, u in ((1.0, 0.0), (0.7, 0.4), (2.5, 0.9999)):
+                gpu.sample_forward(out, x, n, inv_temp, u)
+                assert int(out.item()) == oracle.sample(row, inv_temp, u), (inv_temp, u)
+
+
+def test_sample_forward_overlapping_streams_and_graph(gpu, oracle):
+    """Draws in flight on six streams at once, and a captured draw replayed between eager ones, each
+    equal to the oracle: calls share nothing but the library's slots."""
+    import torch
+    ident("sample_forward on six streams and in a graph")
+    rng = np.random.default_rng(77)
+    n, coins = 151936, [float(c) for c in rng.random(8)]
+    rows = [rand_bf16(rng, n, 2.0) for _ in range(6)]
+    xs = [dev(r) for r in rows]
+    outs = torch.full((6, 8), -7, dtype=torch.int32, device="cuda")
+    streams = [torch.cuda.Stream() for _ in range(6)]
+    want = [[oracle.sample(r, 0.8, c) for c in coins] for r in rows]
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(streams[0]):
+        graph.capture_begin()
+        gpu.sample_forward(outs[0, 0:], xs[0], n, 0.8, coins[0])
+        graph.capture_end()
+    for _ in range(3):
+        outs.fill_(-7)
+        torch.cuda.synchronize()
+        for j, c in enumerate(coins):
+            for i, s in enumerate(streams):
+                if (i, j) != (0, 0):
+                    gpu.sample_forward(outs[i, j:], xs[i], n, 0.8, c, stream=s)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert outs.cpu().tolist() == want
+
+
 # ---------------------------------------------------------------- argmax
 
 def test_argmax(gpu, oracle):
