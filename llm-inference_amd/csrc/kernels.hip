@@ -900,7 +900,23 @@ struct AttnArgs {
     const int *d_pos;
     int n_heads, n_kv_heads, max_seq, max_blocks;
     float scale;
+    int mark;    // the scores pass marks the item's partials as not yet written (ATT_UNWRITTEN)
+    int *err;    // the step's error flag (set to 2 when a wait times out), or NULL
 };
+
+// A block partial that attn_pv_combine_kernel has not stored yet: a NaN that no sum of products of
+// bf16 values produces (a NaN made from bf16 inputs has a payload with a zero low half); should one
+// appear all the same, it is stored as the NaN next to it.
+constexpr uint32_t ATT_UNWRITTEN = 0xffffffffu;
+
+// Marks the partials of block b of the kv head's REP query heads.
+template <int D, int REP>
+__device__ __forceinline__ void mark_partials(const AttnArgs &a, int b, int g) {
+    constexpr int Q = D / 4;  // 16-byte stores per head
+    for (int i = threadIdx.x; i < REP * Q; i += 256)
+        st16(a.partial + ((size_t)(g * REP + i / Q) * a.max_blocks + b) * D + 4 * (i % Q),
+             u32x4{ATT_UNWRITTEN, ATT_UNWRITTEN, ATT_UNWRITTEN, ATT_UNWRITTEN});
+}
 
 static size_t ceil_div(size_t a, size_t b) { return (a + b - 1) / b; }
 
@@ -965,6 +981,7 @@ __global__ __launch_bounds__(256) void attn_scores_kernel(AttnArgs a) {
             }
         }
         __syncthreads();
+        if (a.mark) mark_partials<D, REP>(a, b, g);
         for (int r = w; r < REP; r += 4) {
             const bool v = b * ATT_B + lane < n;
             const float s = v ? sc[r][lane] : -__builtin_huge_valf();
@@ -1193,6 +1210,7 @@ void attn_rope_scores_kernel(AttnRopeArgs r) {
             }
         }
         __syncthreads();
+        if (a.mark) mark_partials<D, REP>(a, b, g);
         for (int q = w; q < REP; q += 4) {
             const bool v = b * ATT_B + lane < n;
             const float s = v ? sc[q][lane] : -__builtin_huge_valf();
@@ -1963,127 +1981,139 @@ extern "C" void qk_norm_rope_attention_one_pass(bf16 *out, const bf16 *q, const 
 }
 
 // ------------------------------------------------------------------------------------------
-// Passes 2 and 3 in one launch (attn_pv_kernel followed by attn_combine_kernel, the same bits),
-// for the step's attention. Every item publishes its block partials as tagged 64-bit words
-// (float bits << 32 | tag; the tag is the workgroup's launch count + 1, counted in a word of
-// its own as in the one-pass kernel), and the items of the T last blocks of each kv head then
-// combine: item nb - T + j adds, in block order, the partials of columns [j C, (j + 1) C) of the
-// kv head's REP * D (C = REP * D / T), once it has read every block's partial of them with the
-// current tag. T is the largest power of two <= min(nb, REP * D / PVC_COLS). One workgroup per
-// item of the longest history, so the items of a step are one wave of the grid; only the
-// T * n_kv_heads combine items wait, every other item runs to its end, so the waits end. They
-// are bounded all the same: a timeout sets *err, and the kernel finishes with what it read.
+// Passes 2 and 3 in one launch (attn_pv_kernel followed by attn_combine_kernel, the same bits).
+// The scores pass has marked every block's partials ATT_UNWRITTEN; every item stores its block
+// partials with agent scope, and the items of the T last blocks of each kv head then combine: item
+// nb - T + j adds, in block order, the partials of columns [j C, (j + 1) C) of the kv head's REP * D
+// (C = REP * D / T), polling the words until none is marked. T is the largest power of two <=
+// min(nb, REP * D / PVC_COLS, PVC_MAX_WAIT / n_kv_heads). The mark travels in the word itself and is
+// set by the launch before, so nothing is counted or kept from call to call, and the words stay 32
+// bits wide. One workgroup per item of the longest history; only the T * n_kv_heads combine items
+// wait, fewer than the workgroups the device holds at once, and every other item runs to its end,
+// so the waits end. They are bounded all the same: on a timeout the kernel finishes with what it
+// read (NaN), and sets *err where there is one.
+//
+// Bound by its chain (statistics, exponentials, the products, the hand-over, the in-order sums)
+// rather than by the value stream: 32 heads on 8 kv heads of 128 at 8300 positions (17 MB of values)
+// 10.6 us, against 8.1 + 5.4 us as two launches; 16 on 8 at 260 positions 5.0 against 3.9 + 3.0; 8 on
+// 4 of 64 at 12345 positions 8.6 against 5.1 + 6.9. In the hipGraph step it replaces a form whose
+// partials were tagged 64-bit words with a launch counter per workgroup, at head_dim 128 only:
+// Qwen3-0.6B after 300 positions 754 -> 730 us per token, 4B after 8192 2276 -> 2268, 8 on 4 heads
+// of 64 after 300 positions (12 layers of 512) 258 -> 243.
 // ------------------------------------------------------------------------------------------
 
 // fewest columns of a combine item (4B after 8192 positions: 431.2-431.8 tokens/s; 8 columns
 // 428.5-428.8, 32 columns 418.5-418.6)
 constexpr int PVC_COLS = 16;
-constexpr int PVC_STRIDE = 16;      // 8-byte words between two workgroups' launch counters
+constexpr int PVC_MAX_WAIT = 512;   // combine items of a launch (the device holds >= 1024 workgroups)
 constexpr int PVC_MAXGRID = 8192;   // items (blocks x kv heads) of the longest history
 
-struct PvCombineArgs {
-    AttnArgs a;
-    unsigned long long *tpart;     // [n_heads, max_blocks, D] tagged block partials
-    unsigned long long *launches;  // per workgroup, PVC_STRIDE words apart: its launches
-    int *err;                      // set to 2 when a wait times out
-};
-
 template <int D, int REP>
-__global__ __launch_bounds__(256) void attn_pv_combine_kernel(PvCombineArgs o) {
+__global__ __launch_bounds__(256) void attn_pv_combine_kernel(AttnArgs a) {
     constexpr int COLS = REP * D;
     constexpr int STAGE = 4 * REP * D > 4096 ? 4 * REP * D : 4096;  // floats
     constexpr int CPT = (COLS + 255) / 256;  // columns of a thread when one item combines all
+    constexpr int K = 4;                     // 16-byte words of a thread in flight while polling
     __shared__ float p_s[REP][ATT_B];
-    __shared__ float stage[STAGE];  // the PV quarter sums, then the combine's staged partials
+    __shared__ __align__(16) float stage[STAGE];  // the PV quarter sums, then the staged partials
     float(&red)[4][REP][D] = *reinterpret_cast<float(*)[4][REP][D]>(stage);
-    const AttnArgs &a = o.a;
-    unsigned long long *ctr = o.launches + (size_t)blockIdx.x * PVC_STRIDE;
-    const unsigned long long launches = op_ld(ctr);
-    const uint32_t tag = (uint32_t)(launches % 0xffffffffull) + 1u;
     const int n = *a.d_pos + 1;
     const int nb = (n + ATT_B - 1) / ATT_B;
-    if (n <= 0 || n > a.max_seq) {  // every workgroup reads the same position: all skip
-        if (threadIdx.x == 0) {
-            __hip_atomic_store(gptr(o.err), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(gptr(ctr), launches + 1, __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-        }
+    if (n <= 0 || n > a.max_seq) {  // no history, or none the caches can hold: zeros
+        if (a.err && threadIdx.x == 0)
+            __hip_atomic_store(gptr(a.err), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if ((int)blockIdx.x < a.n_kv_heads)
+            for (int i = threadIdx.x; i < COLS; i += 256) a.out[(size_t)blockIdx.x * COLS + i] = 0;
         return;
     }
-    if ((int)blockIdx.x < nb * a.n_kv_heads) {  // the grid holds every item: one each
-        const int b = blockIdx.x / a.n_kv_heads, g = blockIdx.x - b * a.n_kv_heads;
-        pv_item<D, REP>(a, b, g, n, nb, p_s, red,
-                        [&](size_t i, float v) { op_st(o.tpart + i, v, tag); });
-        int T = 1;
-        while (2 * T <= nb && 2 * T * PVC_COLS <= COLS) T *= 2;
-        if (b >= nb - T) {
-            const int nc = COLS / T, c0 = (b - (nb - T)) * nc;
-            const int cb = STAGE / nc;  // blocks per staged chunk
-            float acc[CPT];
+    if ((int)blockIdx.x >= nb * a.n_kv_heads) return;  // the grid holds every item: one each
+    const int b = blockIdx.x / a.n_kv_heads, g = blockIdx.x - b * a.n_kv_heads;
+    pv_item<D, REP>(a, b, g, n, nb, p_s, red, [&](size_t i, float v) {
+        const uint32_t u = __float_as_uint(v);
+        __hip_atomic_store(gptr((uint32_t *)a.partial + i), u == ATT_UNWRITTEN ? u - 1 : u,
+                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    });
+    int T = 1;
+    while (2 * T <= nb && 2 * T * PVC_COLS <= COLS && 2 * T * a.n_kv_heads <= PVC_MAX_WAIT) T *= 2;
+    if (b < nb - T) return;
+    const int nc = COLS / T, c0 = (b - (nb - T)) * nc, nq = nc / 4;  // powers of two
+    const int cb = STAGE / nc;                                       // blocks per staged chunk
+    const int qsh = __builtin_ctz(nq);
+    // the kv head's partials as one buffer: REP heads of max_blocks rows of D
+    const __amdgpu_buffer_rsrc_t pr = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(a.partial + (size_t)g * REP * a.max_blocks * D), (short)0,
+        REP * a.max_blocks * D * 4, BUFFER_FLAGS);
+    float acc[CPT];
 #pragma unroll
-            for (int k = 0; k < CPT; k++) acc[k] = 0.0f;
-            for (int b0 = 0; b0 < nb; b0 += cb) {
-                const int cnt = min(cb, nb - b0);
-                op_poll<256, 16>(
-                    cnt * nc, tag, o.err,
-                    [&](int idx) {
-                        const int bb = idx / nc, c = c0 + idx - bb * nc, q = c / D, d = c - q * D;
-                        return o.tpart + ((size_t)(g * REP + q) * a.max_blocks + b0 + bb) * D + d;
-                    },
-                    [&](int idx, float v) { stage[idx] = v; });
-                __syncthreads();
+    for (int k = 0; k < CPT; k++) acc[k] = 0.0f;
+    for (int b0 = 0; b0 < nb; b0 += cb) {
+        const int cnt = min(cb, nb - b0), total = cnt << qsh;
+        for (int base = 0; base < total; base += 256 * K) {
+            u32x4 v[K];
+            int off[K];
 #pragma unroll
-                for (int k = 0; k < CPT; k++) {
-                    const int c = threadIdx.x + 256 * k;
-                    if (c < nc) {
-                        int j0 = 0;
-                        if (b0 == 0) {
-                            acc[k] = stage[c];
-                            j0 = 1;
-                        }
-                        for (; j0 + 16 <= cnt; j0 += 16) {  // 16 LDS reads in flight, then adds
-                            float v[16];
+            for (int k = 0; k < K; k++) {
+                // word quad i: block b0 + i / nq, columns c0 + 4 (i % nq) .. + 3 (past the end: the
+                // last quad again)
+                const int i = min(base + (int)threadIdx.x + 256 * k, total - 1);
+                const int c = c0 + 4 * (i & (nq - 1)), q = c / D;
+                off[k] = ((q * a.max_blocks + b0 + (i >> qsh)) * D + c - q * D) * 4;
+            }
+            long long spins = 0;
+            for (;;) {
+                bool fresh = true;
 #pragma unroll
-                            for (int u = 0; u < 16; u++) v[u] = stage[(j0 + u) * nc + c];
+                for (int k = 0; k < K; k++)
+                    v[k] = __builtin_amdgcn_raw_buffer_load_b128(pr, off[k], 0, BUFFER_SC1);
 #pragma unroll
-                            for (int u = 0; u < 16; u++) acc[k] += v[u];
-                        }
-                        for (; j0 < cnt; j0++) acc[k] += stage[j0 * nc + c];
-                    }
-                }
-                __syncthreads();
+                for (int k = 0; k < K; k++)
+                    fresh &= v[k].x != ATT_UNWRITTEN && v[k].y != ATT_UNWRITTEN &&
+                             v[k].z != ATT_UNWRITTEN && v[k].w != ATT_UNWRITTEN;
+                if (fresh) break;
+                if ((++spins & 15) == 0 &&
+                    (a.err ? wait_gives_up(spins, OP_SPIN_LIMIT, a.err) : spins > OP_SPIN_LIMIT))
+                    break;
+                asm volatile("" ::: "memory");  // read the words again
             }
 #pragma unroll
-            for (int k = 0; k < CPT; k++) {
-                const int c = c0 + threadIdx.x + 256 * k, q = c / D, d = c - q * D;
-                if ((int)threadIdx.x + 256 * k < nc)
-                    a.out[(size_t)(g * REP + q) * D + d] = (bf16)f2bf(acc[k]);
+            for (int k = 0; k < K; k++) {
+                const int i = base + (int)threadIdx.x + 256 * k;
+                if (i < total) *(u32x4 *)(stage + 4 * i) = v[k];
             }
         }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < CPT; k++) {
+            const int c = threadIdx.x + 256 * k;
+            if (c < nc) {
+                int j0 = 0;
+                if (b0 == 0) {
+                    acc[k] = stage[c];
+                    j0 = 1;
+                }
+                for (; j0 + 16 <= cnt; j0 += 16) {  // 16 LDS reads in flight, then adds
+                    float v[16];
+#pragma unroll
+                    for (int u = 0; u < 16; u++) v[u] = stage[(j0 + u) * nc + c];
+#pragma unroll
+                    for (int u = 0; u < 16; u++) acc[k] += v[u];
+                }
+                for (; j0 < cnt; j0++) acc[k] += stage[j0 * nc + c];
+            }
+        }
+        __syncthreads();
     }
-    __syncthreads();  // every wave has its tag
-    if (threadIdx.x == 0)
-        __hip_atomic_store(gptr(ctr), launches + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int k = 0; k < CPT; k++)
+        if ((int)threadIdx.x + 256 * k < nc)
+            a.out[(size_t)g * COLS + c0 + threadIdx.x + 256 * k] = (bf16)f2bf(acc[k]);
 }
 
-// Bytes of the attn_pv_combine_kernel workspace (the launch counters, then the tagged partials),
-// or 0 where that kernel is not used: head_dim other than 128, or more than PVC_MAXGRID items.
-size_t attention_pv_combine_bytes(int n_heads, int n_kv_heads, int head_dim, int max_seq) {
-    if (head_dim != 128 || n_kv_heads <= 0 || n_heads % n_kv_heads != 0 || max_seq <= 0) return 0;
-    const int rep = n_heads / n_kv_heads;
-    if (rep != 1 && rep != 2 && rep != 4 && rep != 8) return 0;
-    const size_t mb = ceil_div((size_t)max_seq, ATT_B);
-    if (mb * n_kv_heads > PVC_MAXGRID) return 0;
-    return mb * n_kv_heads * PVC_STRIDE * 8 + (size_t)n_heads * mb * head_dim * 8;
-}
-
-// The second and third passes: attn_pv_combine_kernel on the workspace `pvc` where given (grid
-// = every item of the longest history, as attention_pv_combine_bytes admits), else the PV and
-// combine kernels.
+// The scores pass, then PV and combine: one launch where the grid holds every item of the longest
+// history (a.mark, set by attention_args), else the two kernels.
 template <int D, int REP>
 static void launch_attention_t(const AttnArgs &a, int grid, hipStream_t stream,
-                               const AttnRopeArgs *rope = nullptr, void *pvc = nullptr,
-                               int *err = nullptr) {
+                               const AttnRopeArgs *rope = nullptr) {
     if (rope && rope->table)
         attn_rope_scores_kernel<D, REP, true><<<grid, 256, 0, stream>>>(*rope);
     else if (rope)
@@ -2091,17 +2121,10 @@ static void launch_attention_t(const AttnArgs &a, int grid, hipStream_t stream,
     else
         attn_scores_kernel<D, REP><<<grid, 256, 0, stream>>>(a);
     if (!LAUNCH_OK()) return;
-    if constexpr (D == 128) {
-        if (pvc) {
-            PvCombineArgs o;
-            o.a = a;
-            o.launches = (unsigned long long *)pvc;
-            o.tpart = o.launches + (size_t)grid * PVC_STRIDE;
-            o.err = err;
-            attn_pv_combine_kernel<D, REP><<<grid, 256, 0, stream>>>(o);
-            LAUNCH_OK();
-            return;
-        }
+    if (a.mark) {
+        attn_pv_combine_kernel<D, REP><<<grid, 256, 0, stream>>>(a);
+        LAUNCH_OK();
+        return;
     }
     attn_pv_kernel<D, REP><<<grid, 256, 0, stream>>>(a);
     if (!LAUNCH_OK()) return;
@@ -2177,7 +2200,7 @@ static bool attention_blocks(float *att, int n_heads, int head_dim, int max_seq,
 static bool attention_args(AttnArgs &a, int &grid, bf16 *out, const bf16 *q,
                            const bf16 *key_cache, const bf16 *value_cache, float *att,
                            int n_heads, int n_kv_heads, int head_dim, const int *d_pos,
-                           int max_seq, float scale) {
+                           int max_seq, float scale, int *err) {
     if (head_dim != 64 && head_dim != 128 && head_dim != 256)
         return llm_fail("attention: head_dim %d is not 64, 128 or 256", head_dim);
     if (n_kv_heads <= 0 || n_heads % n_kv_heads != 0)
@@ -2208,25 +2231,25 @@ static bool attention_args(AttnArgs &a, int &grid, bf16 *out, const bf16 *q,
     // the same wave of workgroups (a fixed cap made the last few items of a long history a second
     // wave that doubled the kernel time); items beyond the current history exit at once
     const long items = (long)a.max_blocks * n_kv_heads;
-    grid = (int)(items < 8192 ? items : 8192);
+    grid = (int)(items < PVC_MAXGRID ? items : PVC_MAXGRID);
+    a.mark = items <= PVC_MAXGRID;
+    a.err = err;
     return true;
 }
 
 bool attention_launch(bf16 *out, const bf16 *q, const bf16 *key_cache, const bf16 *value_cache,
                       float *att, int n_heads, int n_kv_heads, int head_dim, const int *d_pos,
-                      int max_seq, float scale, hipStream_t stream, void *pvc, int *err) {
+                      int max_seq, float scale, hipStream_t stream, int *err) {
     AttnArgs a;
     int grid = 0;
     if (!attention_args(a, grid, out, q, key_cache, value_cache, att, n_heads, n_kv_heads,
-                        head_dim, d_pos, max_seq, scale))
+                        head_dim, d_pos, max_seq, scale, err))
         return false;
-    if (pvc && (!err || !attention_pv_combine_bytes(n_heads, n_kv_heads, head_dim, max_seq)))
-        return llm_fail("attention: no one-launch PV and combine for these shapes");
     const int rep = n_heads / n_kv_heads;
-#define ATT(D_, R_)                                                        \
-    if (head_dim == D_ && rep == R_) {                                     \
-        launch_attention_t<D_, R_>(a, grid, stream, nullptr, pvc, err);    \
-        return !llm_has_error();                                           \
+#define ATT(D_, R_)                               \
+    if (head_dim == D_ && rep == R_) {            \
+        launch_attention_t<D_, R_>(a, grid, stream); \
+        return !llm_has_error();                  \
     }
     ATT(64, 1) ATT(64, 2) ATT(64, 4) ATT(64, 8) ATT(128, 1) ATT(128, 2) ATT(128, 4) ATT(128, 8)
     ATT(256, 1) ATT(256, 2) ATT(256, 4) ATT(256, 8)
@@ -2239,7 +2262,7 @@ extern "C" void attention_forward(bf16 *out, const bf16 *q, const bf16 *key_cach
                                   int head_dim, const int *d_pos, int max_seq, float scale,
                                   hipStream_t stream) {
     attention_launch(out, q, key_cache, value_cache, att, n_heads, n_kv_heads, head_dim, d_pos,
-                     max_seq, scale, stream, nullptr, nullptr);
+                     max_seq, scale, stream);
 }
 
 // Workspace of attention_forward_noalloc: a library-owned device array instead of the caller's
@@ -2276,15 +2299,13 @@ bool qk_norm_rope_attention_launch(bf16 *out, const bf16 *q, const bf16 *k, cons
                                    bf16 *value_cache, float *att, const int *d_pos, int n_heads,
                                    int n_kv_heads, int head_dim, float eps, float theta,
                                    int max_seq, float scale, hipStream_t stream,
-                                   const float *rope_table, void *pvc, int *err) {
+                                   const float *rope_table, int *err) {
     AttnRopeArgs r;
     memset(&r, 0, sizeof r);
     int grid = 0;
     if (!attention_args(r.at, grid, out, q, key_cache, value_cache, att, n_heads, n_kv_heads,
-                        head_dim, d_pos, max_seq, scale))
+                        head_dim, d_pos, max_seq, scale, err))
         return false;
-    if (pvc && (!err || !attention_pv_combine_bytes(n_heads, n_kv_heads, head_dim, max_seq)))
-        return llm_fail("qk_norm_rope_attention: no one-launch PV and combine for these shapes");
     const void *ptrs[] = {k, v, q_norm_w, k_norm_w};
     for (const void *p : ptrs)
         if (!p || !aligned16(p))
@@ -2302,7 +2323,7 @@ bool qk_norm_rope_attention_launch(bf16 *out, const bf16 *q, const bf16 *k, cons
     const int rep = n_heads / n_kv_heads;
 #define ATT(D_, R_)                                        \
     if (head_dim == D_ && rep == R_) {                     \
-        launch_attention_t<D_, R_>(r.at, grid, stream, &r, pvc, err);\
+        launch_attention_t<D_, R_>(r.at, grid, stream, &r);          \
         return !llm_has_error();                                     \
     }
     ATT(64, 1) ATT(64, 2) ATT(64, 4) ATT(64, 8) ATT(128, 1) ATT(128, 2) ATT(128, 4) ATT(128, 8)

@@ -358,6 +358,43 @@ def test_attention_head_dims(gpu, oracle, D, rep):
                                              oracle.EXACT)).max() <= 2
 
 
+# combine widths: one item per kv head (nb = 1), every column count down to 16, the cap on waiting
+# items (REP 8 of 256), two staged chunks of partials, and more items than one launch takes (8200)
+@pytest.mark.parametrize("hq,hkv,D,pos,max_seq", [
+    (2, 2, 64, 5, 64), (16, 2, 64, 700, 704), (4, 4, 256, 127, 128), (8, 8, 64, 17000, 17001),
+    (64, 8, 256, 8200, 8256), (8, 1, 128, 9000, 9001), (8, 8, 64, 1000, 65600), (4, 4, 128, -1, 200)])
+def test_attention_one_launch_combine(gpu, oracle, hq, hkv, D, pos, max_seq):
+    """The PV pass and the combine in one launch: bit-identical to the oracle whatever `att` held
+    before (the mark of an unwritten partial, another call's partials), at a later and an earlier
+    position on the same workspace, and with NaN among the values. Position -1 (no history) gives
+    zeros."""
+    import torch
+    ident(f"attention one-launch combine {hq}/{hkv} D{D} pos{pos} of {max_seq}")
+    rng = np.random.default_rng(hq * 1000 + pos)
+    kc = rand_bf16(rng, (max_seq, hkv * D))
+    vc = rand_bf16(rng, (max_seq, hkv * D))
+    floats = gpu.attention_workspace_floats(hq, D, max_seq)
+    att = torch.full((floats,), -1, dtype=torch.int32, device="cuda").view(torch.float32)
+    out = dev(np.full(hq * D, 0x1234, np.uint16))
+    scale = float(np.float32(1.0 / np.sqrt(D)))
+    kd, vd = dev(kc), dev(vc)
+    for p in (pos, pos // 3, pos):
+        q = rand_bf16(rng, hq * D)
+        gpu.attention_forward(out, dev(q), kd, vd, att, hq, hkv, D, dev_i32([p]), max_seq, scale)
+        want = (oracle.attention(q, kc, vc, hq, hkv, D, p, scale, oracle.GPU_ORDER) if p >= 0
+                else np.zeros(hq * D, np.uint16))
+        assert np.array_equal(host(out), want), p
+    if pos < 0:
+        return
+    vc[pos // 2, 1], vc[pos // 2, 2] = 0xFFFF, 0x7FFF  # NaNs with every payload bit set
+    gpu.attention_forward(out, dev(q), kd, dev(vc), att, hq, hkv, D, dev_i32([pos]), max_seq, scale)
+    got, rep = host(out).copy(), hq // hkv
+    nan = np.isnan(bf16_vals(got)).reshape(hq, D)
+    assert nan[:rep, 1:3].all() and nan.sum() == 2 * rep
+    got.reshape(hq, D)[:rep, 1:3] = want.reshape(hq, D)[:rep, 1:3]
+    assert np.array_equal(got, want)
+
+
 FUSED_ATTN_CASES = [(16, 8, 128, 0, 4096), (16, 8, 128, 63, 4096), (16, 8, 128, 64, 4096),
                     (16, 8, 128, 260, 4096), (32, 8, 128, 8192, 8448), (32, 8, 128, 8447, 8448),
                     (8, 8, 128, 100, 512), (8, 1, 128, 130, 512), (2, 2, 64, 301, 512),
