@@ -152,8 +152,86 @@ __global__ __launch_bounds__(256) void rmsnorm_wave_kernel(bf16 *out, const bf16
     }
 }
 
-// Any dim: W waves per row (W = max(1, min(16, ceil(chunks / 1024)))), thread t takes chunks
-// t, t + 64W, ... element by element; wave trees, then the waves added in order through LDS.
+// Rows that rmsnorm_wave_kernel does not take: wider than 8192, of a dim that is no multiple of 8,
+// or not 16-byte aligned. T threads per row (64 W, W = max(1, min(16, ceil(chunks / 1024))); four rows
+// per workgroup when W = 1), thread t holds chunks t, t + T, ... (NC of them) in registers and sums
+// its squares in chunk/element order; the dim % 8 elements behind the last whole chunk belong to the
+// thread that chunk index falls to, last in its order. Wave trees, then the waves added in order
+// through LDS. Chunks past the row are the last one read again and left out of the sum, and the
+// elements behind the chunks come from the row's last 8, so no branch surrounds a load.
+//
+// Bound by memory: 16-byte accesses at whatever element the row begins (rows of odd dims cross more
+// cache lines than those that begin on a multiple of 4 or 16 bytes). The element-by-element form it
+// replaces read each row twice with a bounds test per element: 1000 x 9000 31.0 -> 7.4 us (4.9 TB/s),
+// 1000 x 9001 32.2 -> 9.2, 4096 x 8190 80.3 -> 27.5, 4096 x 2561 26.9 -> 10.5, 1 x 9000 16.8 -> 3.4,
+// 4096 x 101 3.9 -> 3.8. Up to two chunks per thread the stores are plain: such rows end inside cache
+// lines that others begin in (4096 x 101 4.2 us with non-temporal ones, 4096 x 1025 5.7 against 5.5;
+// 1000 x 9000 8.4 with plain ones).
+template <int NC, int THREADS>
+__global__ __launch_bounds__(THREADS) void rmsnorm_rows_kernel(bf16 *out, const bf16 *in,
+                                                               const bf16 *weight, int rows,
+                                                               int dim, int waves, float eps) {
+    typedef u32x4 chunk_t __attribute__((aligned(2)));  // 16 bytes at an element boundary
+    __shared__ float part[16];
+    const bool alone = waves == 1;  // a wave per row, four rows per workgroup: no sync
+    const int T = 64 * waves;
+    const int t = alone ? (int)(threadIdx.x & 63) : (int)threadIdx.x;
+    const int row = alone ? (int)blockIdx.x * 4 + wave_id() : (int)blockIdx.x;
+    if (row >= rows) return;
+    const LLM_GLOBAL bf16 *x = gptr(in + (size_t)row * dim), *g = gptr(weight);
+    LLM_GLOBAL bf16 *y = gptr(out + (size_t)row * dim);
+    const int full = dim >> 3, rem = dim & 7;  // whole chunks (at least one), elements behind them
+    u32x4 xv[NC], wv[NC];
+#pragma unroll
+    for (int k = 0; k < NC; k++)
+        xv[k] = __builtin_nontemporal_load(
+            (const LLM_GLOBAL chunk_t *)(x + 8 * min(t + T * k, full - 1)));
+    const u32x4 xl = *(const LLM_GLOBAL chunk_t *)(x + dim - 8);  // the row's last 8 elements
+    // the weights with the row, or where 16 waves' registers do not hold both, at their use
+    constexpr bool EARLY = THREADS <= 256;
+    const auto weights = [&](int k) {
+        return (u32x4)*(const LLM_GLOBAL chunk_t *)(g + 8 * min(t + T * k, full - 1));
+    };
+#pragma unroll
+    for (int k = 0; k < NC && EARLY; k++) wv[k] = weights(k);
+    const u32x4 wl = *(const LLM_GLOBAL chunk_t *)(g + dim - 8);
+    const bool tail = rem != 0 && t == full % T;
+    float acc = 0.0f;
+#pragma unroll
+    for (int k = 0; k < NC; k++) {
+        const float sum = dot8(xv[k], xv[k], acc);
+        acc = t + T * k < full ? sum : acc;
+    }
+#pragma unroll
+    for (int e = 1; e < 8; e++) {
+        const float sum = fmaf(elem(xl, e), elem(xl, e), acc);
+        acc = tail && e >= 8 - rem ? sum : acc;
+    }
+    float total = wave_sum(acc);
+    if (!alone) {
+        if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = total;
+        __syncthreads();
+        total = part[0];
+        for (int w = 1; w < waves; w++) total = total + part[w];
+    }
+    const float inv = 1.0f / sqrtf(total / (float)dim + eps);
+    const auto store = [&](int at, const u32x4 &xc, const u32x4 &wc) {
+        float r[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) r[e] = round_bf(elem(xc, e) * inv) * elem(wc, e);
+        const u32x4 v{pack2(r[0], r[1]), pack2(r[2], r[3]), pack2(r[4], r[5]), pack2(r[6], r[7])};
+        if constexpr (NC <= 2)
+            *(LLM_GLOBAL chunk_t *)(y + at) = v;
+        else
+            __builtin_nontemporal_store(v, (LLM_GLOBAL chunk_t *)(y + at));
+    };
+#pragma unroll
+    for (int k = 0; k < NC; k++)
+        if (t + T * k < full) store(8 * (t + T * k), xv[k], EARLY ? wv[k] : weights(k));
+    if (tail) store(dim - 8, xl, wl);  // over elements of the last chunk too: the same values
+}
+
+// The rest (dim < 8, or over 16 chunks per thread: dim > 131072): the same sums, element by element.
 __global__ __launch_bounds__(1024) void rmsnorm_generic_kernel(bf16 *out, const bf16 *in,
                                                                const bf16 *weight, int dim,
                                                                float eps) {
@@ -208,7 +286,22 @@ extern "C" void rmsnorm_forward(bf16 *out, const bf16 *in, const bf16 *weight, i
         RMS(1) RMS(2) RMS(3) RMS(4) RMS(5) RMS(6) RMS(8) RMS(12) RMS(16)
 #undef RMS
     }
-    rmsnorm_generic_kernel<<<rows, 64 * rms_waves(dim), 0, stream>>>(out, in, weight, dim, eps);
+    const int waves = rms_waves(dim), held = (dim / 8 + 64 * waves - 1) / (64 * waves);
+    if (dim >= 8 && held <= 16) {
+        // over 4 waves a row has more than 12 chunks per thread
+        const int blocks = waves == 1 ? (rows + 3) / 4 : rows, threads = waves == 1 ? 256 : 64 * waves;
+#define RMS(NC_, THREADS_)                                                                     \
+    if (held <= NC_ && threads <= THREADS_) {                                                  \
+        rmsnorm_rows_kernel<NC_, THREADS_>                                                     \
+            <<<blocks, threads, 0, stream>>>(out, in, weight, rows, dim, waves, eps);          \
+        LAUNCH_OK();                                                                           \
+        return;                                                                                \
+    }
+        RMS(1, 256) RMS(2, 256) RMS(4, 256) RMS(6, 256) RMS(8, 256) RMS(10, 256) RMS(12, 256)
+        RMS(16, 256) RMS(16, 1024)
+#undef RMS
+    }
+    rmsnorm_generic_kernel<<<rows, 64 * waves, 0, stream>>>(out, in, weight, dim, eps);
     LAUNCH_OK();
 }
 

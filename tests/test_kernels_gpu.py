@@ -68,6 +68,32 @@ def test_rmsnorm(gpu, oracle, rows, dim):
     assert within_one_ulp_then_scale(y, n_exact, w).all()
 
 
+# one chunk and a tail, the last whole chunk of a wave, one to two waves (8192), two to five, the
+# widest held in registers (131079) and the next row that is not; element offsets of the buffers
+@pytest.mark.parametrize("dim", [7, 9, 15, 511, 513, 1023, 5000, 8191, 8193, 8200, 9001, 16384, 16391,
+                                 32773, 131079, 131080])
+@pytest.mark.parametrize("offset", [0, 1, 4])
+def test_rmsnorm_row_forms(gpu, oracle, dim, offset):
+    """Rows of any width at any element alignment, also in place, equal the oracle; the elements
+    around the output stay."""
+    import torch
+    ident(f"rmsnorm rows of {dim} at element {offset}")
+    rows = 5
+    rng = np.random.default_rng(dim + offset)
+    x, w = rand_bf16(rng, (rows, dim)), rand_bf16(rng, dim, 0.1, 1.0)
+    pad = np.zeros(offset, np.uint16)
+    xd = dev(np.concatenate([pad, x.reshape(-1), [0x7FC0] * 8]))
+    wd = dev(np.concatenate([pad, w, [0x7FC0] * 8]))
+    out = torch.full((offset + rows * dim + 8,), 0x1234, dtype=torch.int16, device="cuda")
+    want = oracle.rmsnorm(x, w, 1e-6, oracle.GPU_ORDER).reshape(-1)
+    gpu.rmsnorm_forward(out[offset:], xd[offset:], wd[offset:], rows, dim, 1e-6)
+    got = host(out)
+    assert np.array_equal(got[offset:offset + rows * dim], want)
+    assert (got[:offset] == 0x1234).all() and (got[offset + rows * dim:] == 0x1234).all()
+    gpu.rmsnorm_forward(xd[offset:], xd[offset:], wd[offset:], rows, dim, 1e-6)
+    assert np.array_equal(host(xd)[offset:offset + rows * dim], want)
+
+
 # ---------------------------------------------------------------- GEMV family
 
 GEMV_SHAPES = [(4096, 1024), (1024, 2048), (1024, 3072), (2560, 9728), (2560, 4096),
