@@ -4,7 +4,8 @@ Thin ctypes bindings of libllm_amd.so, whose C ABI (include/llm_amd/kernels.h, f
 replaces the reference's src/kernels.cuh and src/forward.cuh launchers and step API
 (William-Lamer/llm-inference). The wrappers take torch tensors for device memory and a torch
 stream (or the current one); torch is only the allocator and stream provider. Every call goes to
-the HIP kernels: there is no CPU path, and a missing library raises.
+the HIP kernels: there is no CPU path, and a missing library raises. The launchers are called
+through a native module (csrc/launchers.cpp), arguments it does not recognise through ctypes.
 
 Errors the reference reports with exit(EXIT_FAILURE) raise LlmError here (the library is
 switched to recording mode on load).
@@ -50,6 +51,7 @@ class LlmError(RuntimeError):
 
 
 _lib = None
+_native = None  # the _launchers module, once the library is loaded
 
 _vp = ctypes.c_void_p
 _i = ctypes.c_int
@@ -94,7 +96,7 @@ _SIGS = {
 
 def lib():
     """The loaded libllm_amd.so (raises LlmError if it has not been built)."""
-    global _lib
+    global _lib, _native
     if _lib is None:
         # torch first: its bundled HIP runtime then satisfies the library's libamdhip64.so.7
         # dependency (same SONAME), so both share one runtime and torch's streams are valid here.
@@ -108,7 +110,13 @@ def lib():
             fn.restype = res
             fn.argtypes = args
         L.llm_set_exit_on_error(0)
-        _lib = L
+        try:
+            from . import _launchers
+        except ImportError as e:
+            raise LlmError(f"{HERE / '_launchers.so'} is missing or does not load ({e}): build it "
+                           f"with `make -C {HERE}` (or __graft_entry__.build())") from e
+        _launchers.init(LlmError)
+        _lib, _native = L, _launchers
         from . import model  # noqa: F401  (declares the step API signatures)
         model._declare(L)
     return _lib
@@ -157,35 +165,49 @@ def _call(fn, *args):
     check()
 
 
-# ---- launchers (include/llm_amd/kernels.h) ----
+# ---- launchers (include/llm_amd/kernels.h): the native module first, the general way for what it
+# does not recognise ----
 
 def embedding_forward(out, table, d_token, hidden, stream=None):
+    if _native and _native.embedding_forward(out, table, d_token, hidden, stream):
+        return
     _call(lib().embedding_forward, _bf16(out, "out"), _bf16(table, "table"), _ptr(d_token),
           hidden, _stream(stream))
 
 
 def rmsnorm_forward(out, inp, weight, rows, dim, eps, stream=None):
+    if _native and _native.rmsnorm_forward(out, inp, weight, rows, dim, eps, stream):
+        return
     _call(lib().rmsnorm_forward, _bf16(out, "out"), _bf16(inp, "in"), _bf16(weight, "weight"),
           rows, dim, eps, _stream(stream))
 
 
 def gemv_forward(out, w, x, rows, cols, stream=None):
+    if _native and _native.gemv_forward(out, w, x, rows, cols, stream):
+        return
     _call(lib().gemv_forward, _bf16(out, "out"), _bf16(w, "w"), _bf16(x, "x"), rows, cols,
           _stream(stream))
 
 
 def gemv_residual_forward(x, w, inp, rows, cols, tap=None, stream=None):
+    if _native and _native.gemv_residual_forward(x, w, inp, rows, cols, tap, stream):
+        return
     _call(lib().gemv_residual_forward, _bf16(x, "x"), _bf16(w, "w"), _bf16(inp, "in"), rows,
           cols, _bf16(tap, "tap"), _stream(stream))
 
 
 def qkv_forward(q, k, v, wq, wk, wv, x, q_rows, kv_rows, cols, stream=None):
+    if _native and _native.qkv_forward(q, k, v, wq, wk, wv, x, q_rows, kv_rows, cols, stream):
+        return
     _call(lib().qkv_forward, _bf16(q, "q"), _bf16(k, "k"), _bf16(v, "v"), _bf16(wq, "wq"),
           _bf16(wk, "wk"), _bf16(wv, "wv"), _bf16(x, "x"), q_rows, kv_rows, cols,
           _stream(stream))
 
 
 def gate_up_forward(act, w_gate, w_up, x, rows, cols, gate_tap=None, up_tap=None, stream=None):
+    if _native and _native.gate_up_forward(act, w_gate, w_up, x, rows, cols, gate_tap, up_tap,
+                                           stream):
+        return
     _call(lib().gate_up_forward, _bf16(act, "act"), _bf16(w_gate, "w_gate"), _bf16(w_up, "w_up"),
           _bf16(x, "x"), rows, cols, _bf16(gate_tap, "gate_tap"), _bf16(up_tap, "up_tap"),
           _stream(stream))
@@ -193,17 +215,25 @@ def gate_up_forward(act, w_gate, w_up, x, rows, cols, gate_tap=None, up_tap=None
 
 def rmsnorm_qkv_forward(q, k, v, wq, wk, wv, x, norm_w, eps, q_rows, kv_rows, cols,
                         stream=None):
+    if _native and _native.rmsnorm_qkv_forward(q, k, v, wq, wk, wv, x, norm_w, eps, q_rows, kv_rows,
+                                               cols, stream):
+        return
     _call(lib().rmsnorm_qkv_forward, _bf16(q, "q"), _bf16(k, "k"), _bf16(v, "v"),
           _bf16(wq, "wq"), _bf16(wk, "wk"), _bf16(wv, "wv"), _bf16(x, "x"),
           _bf16(norm_w, "norm_w"), eps, q_rows, kv_rows, cols, _stream(stream))
 
 
 def rmsnorm_gemv_forward(out, w, x, norm_w, eps, rows, cols, stream=None):
+    if _native and _native.rmsnorm_gemv_forward(out, w, x, norm_w, eps, rows, cols, stream):
+        return
     _call(lib().rmsnorm_gemv_forward, _bf16(out, "out"), _bf16(w, "w"), _bf16(x, "x"),
           _bf16(norm_w, "norm_w"), eps, rows, cols, _stream(stream))
 
 
 def rmsnorm_gate_up_forward(act, w_gate, w_up, x, norm_w, eps, rows, cols, stream=None):
+    if _native and _native.rmsnorm_gate_up_forward(act, w_gate, w_up, x, norm_w, eps, rows, cols,
+                                                   stream):
+        return
     _call(lib().rmsnorm_gate_up_forward, _bf16(act, "act"), _bf16(w_gate, "w_gate"),
           _bf16(w_up, "w_up"), _bf16(x, "x"), _bf16(norm_w, "norm_w"), eps, rows, cols,
           _stream(stream))
@@ -211,6 +241,10 @@ def rmsnorm_gate_up_forward(act, w_gate, w_up, x, norm_w, eps, rows, cols, strea
 
 def qk_norm_rope_forward(q, k, v, q_norm_w, k_norm_w, key_cache, value_cache, d_pos, n_heads,
                          n_kv_heads, head_dim, eps, theta, q_tap=None, k_tap=None, stream=None):
+    if _native and _native.qk_norm_rope_forward(q, k, v, q_norm_w, k_norm_w, key_cache, value_cache,
+                                                d_pos, n_heads, n_kv_heads, head_dim, eps, theta,
+                                                q_tap, k_tap, stream):
+        return
     _call(lib().qk_norm_rope_forward, _bf16(q, "q"), _bf16(k, "k"), _bf16(v, "v"),
           _bf16(q_norm_w, "q_norm_w"), _bf16(k_norm_w, "k_norm_w"), _bf16(key_cache, "key_cache"),
           _bf16(value_cache, "value_cache"), _ptr(d_pos), n_heads, n_kv_heads, head_dim, eps,
@@ -220,6 +254,10 @@ def qk_norm_rope_forward(q, k, v, q_norm_w, k_norm_w, key_cache, value_cache, d_
 def qk_norm_rope_rows(q, k, v, q_norm_w, k_norm_w, key_cache, value_cache, d_positions,
                       n_tokens, n_heads, n_kv_heads, head_dim, eps, theta, q_tap=None,
                       k_tap=None, stream=None):
+    if _native and _native.qk_norm_rope_rows(q, k, v, q_norm_w, k_norm_w, key_cache, value_cache,
+                                             d_positions, n_tokens, n_heads, n_kv_heads, head_dim,
+                                             eps, theta, q_tap, k_tap, stream):
+        return
     _call(lib().qk_norm_rope_rows, _bf16(q, "q"), _bf16(k, "k"), _bf16(v, "v"),
           _bf16(q_norm_w, "q_norm_w"), _bf16(k_norm_w, "k_norm_w"), _bf16(key_cache, "key_cache"),
           _bf16(value_cache, "value_cache"), _ptr(d_positions), n_tokens, n_heads, n_kv_heads,
@@ -236,6 +274,9 @@ def attention_forward(out, q, key_cache, value_cache, att, n_heads, n_kv_heads, 
     floats (the library checks that allocation's size), or a torch tensor of at least
     attention_workspace_floats(n_heads, head_dim, max_seq) floats: torch's caching allocator
     carves tensors out of larger allocations, whose size says nothing of the tensor's."""
+    if _native and _native.attention_forward(out, q, key_cache, value_cache, att, n_heads,
+                                             n_kv_heads, head_dim, d_pos, max_seq, scale, stream):
+        return
     need = attention_workspace_floats(n_heads, head_dim, max_seq)
     if not isinstance(att, int) and att.numel() < need:
         raise LlmError(f"att holds {att.numel()} floats, attention needs {need}")
@@ -248,6 +289,11 @@ def qk_norm_rope_attention_forward(out, q, k, v, q_norm_w, k_norm_w, key_cache, 
                                    d_pos, n_heads, n_kv_heads, head_dim, eps, theta, max_seq,
                                    scale, stream=None):
     """qk_norm_rope_forward + attention_forward, the QK-norm + RoPE inside the scores pass."""
+    if _native and _native.qk_norm_rope_attention_forward(out, q, k, v, q_norm_w, k_norm_w,
+                                                          key_cache, value_cache, att, d_pos,
+                                                          n_heads, n_kv_heads, head_dim, eps, theta,
+                                                          max_seq, scale, stream):
+        return
     need = attention_workspace_floats(n_heads, head_dim, max_seq)
     if not isinstance(att, int) and att.numel() < need:
         raise LlmError(f"att holds {att.numel()} floats, attention needs {need}")
@@ -284,6 +330,10 @@ def qk_norm_rope_attention_one_pass(out, q, k, v, q_norm_w, k_norm_w, key_cache,
 def attention_forward_noalloc(out, q, key_cache, value_cache, n_heads, n_kv_heads, head_dim,
                               d_pos, max_seq, scale, stream=None):
     """attention_forward with the library's own workspace (allocates nothing)."""
+    if _native and _native.attention_forward_noalloc(out, q, key_cache, value_cache, n_heads,
+                                                     n_kv_heads, head_dim, d_pos, max_seq, scale,
+                                                     stream):
+        return
     _call(lib().attention_forward_noalloc, _bf16(out, "out"), _bf16(q, "q"),
           _bf16(key_cache, "key_cache"), _bf16(value_cache, "value_cache"), n_heads, n_kv_heads,
           head_dim, _ptr(d_pos), max_seq, scale, _stream(stream))
@@ -319,6 +369,8 @@ def hbm_copy_peak_probe(dst, a, n_bytes, blocks, threads, chunks_in_flight=4, st
 
 
 def sample_forward(out, x, n, inv_temp, u, stream=None):
+    if _native and _native.sample_forward(out, x, n, inv_temp, u, stream):
+        return
     _call(lib().sample_forward, _ptr(out), _bf16(x, "x"), n, inv_temp, u, _stream(stream))
 
 
@@ -332,9 +384,13 @@ def dump_close():
 
 
 def argmax_forward(out, x, n, stream=None):
+    if _native and _native.argmax_forward(out, x, n, stream):
+        return
     _call(lib().argmax_forward, _ptr(out), _bf16(x, "x"), n, _stream(stream))
 
 
 def swiglu_forward(act, gate, up, n, stream=None):
+    if _native and _native.swiglu_forward(act, gate, up, n, stream):
+        return
     _call(lib().swiglu_forward, _bf16(act, "act"), _bf16(gate, "gate"), _bf16(up, "up"), n,
           _stream(stream))
