@@ -11,6 +11,7 @@
 #include <string.h>
 
 #include <mutex>
+#include <type_traits>
 
 #include "common.h"
 #include "internal.h"
@@ -980,6 +981,27 @@ extern "C" void qk_norm_rope_rows(bf16 *q, bf16 *k, const bf16 *v, const bf16 *q
 // decode attention, split softmax (src/kernels.cu:439-497)
 // ------------------------------------------------------------------------------------------
 
+// 16 consecutive floats of LDS (16-byte aligned), all requested at once.
+__device__ __forceinline__ void ld_lds16(const float *p, float (&v)[16]) {
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    const f32x4 *q = (const f32x4 *)p;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const f32x4 a = q[i];
+        v[4 * i] = a.x;
+        v[4 * i + 1] = a.y;
+        v[4 * i + 2] = a.z;
+        v[4 * i + 3] = a.w;
+    }
+}
+
+__device__ __forceinline__ void st_lds16(float *p, const float (&v)[16]) {
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    f32x4 *q = (f32x4 *)p;
+#pragma unroll
+    for (int i = 0; i < 4; i++) q[i] = f32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
+}
+
 constexpr int ATT_B = 64;  // positions per block
 
 struct AttnArgs {
@@ -1334,15 +1356,15 @@ __device__ __forceinline__ void pv_item(const AttnArgs &a, int b, int g, int n, 
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int G = lane / LP, L = lane % LP;
     const int kv_dim = a.n_kv_heads * D;
-    // The first head of this wave (r = w): its score and block statistics are requested
-    // before the values. Loads complete in order, so the statistics chain then waits only
-    // for them and runs while the values stream. Unconditional (clamped indices), so no
-    // branch joins before the value requests.
+    // The first head of this wave (r = w, where it has one): its score and block statistics are
+    // requested before the values. Loads complete in order, so the statistics chain then waits only
+    // for them and runs while the values stream. Unconditional (clamped indices), so no branch joins
+    // before the value requests.
     constexpr int MAXC = 4;  // chunks of 64 block statistics held in registers
-    const int r_first = w < REP ? w : 0;
+    const int wu = wave_id();
     float mv0[MAXC], sv0[MAXC], s_t0;
     {
-        const int h = g * REP + r_first;
+        const int h = g * REP + (wu < REP ? wu : 0);
         const float *st = a.stats + (size_t)h * a.max_blocks * 2;
         s_t0 = a.scores[(size_t)h * a.max_seq + min(b * ATT_B + lane, n - 1)];
 #pragma unroll
@@ -1360,39 +1382,48 @@ __device__ __forceinline__ void pv_item(const AttnArgs &a, int b, int g, int n, 
         const int t = min(b * ATT_B + w * PER_WAVE + it * PPW + G, n - 1);
         vv[it] = ld16_nt(a.vc + (size_t)t * kv_dim + g * D + 8 * L);
     }
-    // The first head's probabilities from those statistics (nb <= 64 * MAXC: the max is exact
-    // in any order, so over the lane's chunks first and then one wave_max; the chunk sums
-    // added in order), computed by every wave with no branch, so the requests above are not
-    // moved below the value requests. Kept only by a wave that has a head, for nb <= 64 MAXC.
-    float p0;
-    {
+    asm volatile("" ::: "memory");  // the requests stay ahead of the branches below
+    // The probability of this lane's position from its score and the head's block statistics (at
+    // most C chunks of 64). The max is exact in any order, so over the lane's chunks first and then
+    // one wave_max; the chunk sums (wave_sum of each, scattered over the lanes) are added in order.
+    const auto prob = [&](auto chunks, float s_t, const float (&mv)[MAXC], const float (&sv)[MAXC]) {
+        constexpr int C = decltype(chunks)::value, B = C == 3 ? 4 : C;
         float ml = -__builtin_huge_valf();
 #pragma unroll
-        for (int c = 0; c < MAXC; c++) ml = c * 64 + lane < nb ? fmaxf(ml, mv0[c]) : ml;
+        for (int c = 0; c < C; c++) ml = c * 64 + lane < nb ? fmaxf(ml, mv[c]) : ml;
         const float M = wave_max(ml);
-        float cs[MAXC];
+        float term[B];
 #pragma unroll
-        for (int c = 0; c < MAXC; c++)
-            cs[c] = wave_sum(c * 64 + lane < nb ? sv0[c] * exp_f32(mv0[c] - M) : 0.0f);
-        float sum = cs[0];
+        for (int c = 0; c < B; c++)
+            term[c] = c < C && c * 64 + lane < nb ? sv[c] * exp_f32(mv[c] - M) : 0.0f;
+        const float totals = wave_sum_scatter<B>(term);
+        float sum = 0.0f;
 #pragma unroll
-        for (int c = 1; c < MAXC; c++) sum = c * 64 < nb ? sum + cs[c] : sum;
-        p0 = b * ATT_B + lane < n ? round_bf(exp_f32(s_t0 - M) / sum) : 0.0f;
-    }
-    for (int r = w; r < REP; r += 4) {
-        if (r == w && nb <= 64 * MAXC) {
-            p_s[r][lane] = p0;
-            continue;
+        for (int c = 0; c < C; c++) {
+            // chunk c's total is in the lane that scatter_row maps to it
+            const int at = B == 4 ? ((c & 1) << 1 | c >> 1) : c;
+            const float cs = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(totals), at));
+            sum = c == 0 ? cs : sum + cs;
         }
-        // a second head of the wave (REP = 8), or more than 64 * MAXC blocks
-        const int h = g * REP + r;
-        const float *st = a.stats + (size_t)h * a.max_blocks * 2;
-        const int t = b * ATT_B + lane;
-        const float s_t = a.scores[(size_t)h * a.max_seq + min(t, n - 1)];
-        float M = -__builtin_huge_valf(), sum = 0.0f;
+        return b * ATT_B + lane < n ? round_bf(exp_f32(s_t - M) / sum) : 0.0f;
+    };
+    const auto prob_of = [&](float s_t, const float (&mv)[MAXC], const float (&sv)[MAXC]) {
+        if (nb <= 64) return prob(std::integral_constant<int, 1>{}, s_t, mv, sv);
+        if (nb <= 128) return prob(std::integral_constant<int, 2>{}, s_t, mv, sv);
+        if (nb <= 192) return prob(std::integral_constant<int, 3>{}, s_t, mv, sv);
+        return prob(std::integral_constant<int, MAXC>{}, s_t, mv, sv);
+    };
+    static_assert(MAXC == 4, "chunk counts");
+    for (int r = wu; r < REP; r += 4) {
         if (nb <= 64 * MAXC) {
-            // every statistic requested at once (clamped indices, no branch around the
-            // loads), then the same max and in-order chunk sums as p0's
+            if (r == wu) {
+                p_s[r][lane] = prob_of(s_t0, mv0, sv0);
+                continue;
+            }
+            // a second head of the wave (REP = 8): every statistic requested at once
+            const int h = g * REP + r;
+            const float *st = a.stats + (size_t)h * a.max_blocks * 2;
+            const float s_t = a.scores[(size_t)h * a.max_seq + min(b * ATT_B + lane, n - 1)];
             float mv[MAXC], sv[MAXC];
 #pragma unroll
             for (int c = 0; c < MAXC; c++) {
@@ -1400,29 +1431,24 @@ __device__ __forceinline__ void pv_item(const AttnArgs &a, int b, int g, int n, 
                 mv[c] = st[2 * bi];
                 sv[c] = st[2 * bi + 1];
             }
-            float ml = -__builtin_huge_valf();
-#pragma unroll
-            for (int c = 0; c < MAXC; c++)
-                if (c * 64 + lane < nb) ml = fmaxf(ml, mv[c]);
-            M = wave_max(ml);
-#pragma unroll
-            for (int c = 0; c < MAXC; c++)
-                if (c * 64 < nb) {
-                    const float term = c * 64 + lane < nb ? sv[c] * exp_f32(mv[c] - M) : 0.0f;
-                    const float cs = wave_sum(term);
-                    sum = c == 0 ? cs : sum + cs;
-                }
-        } else {
-            for (int c0 = 0; c0 < nb; c0 += 64) {
-                const int bi = c0 + lane;
-                M = fmaxf(M, wave_max(bi < nb ? st[2 * bi] : -__builtin_huge_valf()));
-            }
-            for (int c0 = 0; c0 < nb; c0 += 64) {
-                const int bi = c0 + lane;
-                const float term = bi < nb ? st[2 * bi + 1] * exp_f32(st[2 * bi] - M) : 0.0f;
-                const float cs = wave_sum(term);
-                sum = c0 == 0 ? cs : sum + cs;
-            }
+            p_s[r][lane] = prob_of(s_t, mv, sv);
+            continue;
+        }
+        // more than 64 * MAXC blocks
+        const int h = g * REP + r;
+        const float *st = a.stats + (size_t)h * a.max_blocks * 2;
+        const int t = b * ATT_B + lane;
+        const float s_t = a.scores[(size_t)h * a.max_seq + min(t, n - 1)];
+        float M = -__builtin_huge_valf(), sum = 0.0f;
+        for (int c0 = 0; c0 < nb; c0 += 64) {
+            const int bi = c0 + lane;
+            M = fmaxf(M, wave_max(bi < nb ? st[2 * bi] : -__builtin_huge_valf()));
+        }
+        for (int c0 = 0; c0 < nb; c0 += 64) {
+            const int bi = c0 + lane;
+            const float term = bi < nb ? st[2 * bi + 1] * exp_f32(st[2 * bi] - M) : 0.0f;
+            const float cs = wave_sum(term);
+            sum = c0 == 0 ? cs : sum + cs;
         }
         p_s[r][lane] = t < n ? round_bf(exp_f32(s_t - M) / sum) : 0.0f;
     }
@@ -2130,7 +2156,9 @@ __global__ __launch_bounds__(256) void attn_pv_combine_kernel(AttnArgs a) {
     while (2 * T <= nb && 2 * T * PVC_COLS <= COLS && 2 * T * a.n_kv_heads <= PVC_MAX_WAIT) T *= 2;
     if (b < nb - T) return;
     const int nc = COLS / T, c0 = (b - (nb - T)) * nc, nq = nc / 4;  // powers of two
-    const int cb = STAGE / nc;                                       // blocks per staged chunk
+    // blocks per staged chunk: a column's partials lie side by side (read 16 bytes at a time), the
+    // columns an odd multiple of 16 bytes apart where there is room
+    const int cb = STAGE / nc >= 32 ? STAGE / nc - 4 : STAGE / nc;
     const int qsh = __builtin_ctz(nq);
     // the kv head's partials as one buffer: REP heads of max_blocks rows of D
     const __amdgpu_buffer_rsrc_t pr = __builtin_amdgcn_make_buffer_rsrc(
@@ -2138,7 +2166,7 @@ __global__ __launch_bounds__(256) void attn_pv_combine_kernel(AttnArgs a) {
         REP * a.max_blocks * D * 4, BUFFER_FLAGS);
     float acc[CPT];
 #pragma unroll
-    for (int k = 0; k < CPT; k++) acc[k] = 0.0f;
+    for (int k = 0; k < CPT; k++) acc[k] = -0.0f;  // -0 + x is x, also for x = -0
     for (int b0 = 0; b0 < nb; b0 += cb) {
         const int cnt = min(cb, nb - b0), total = cnt << qsh;
         for (int base = 0; base < total; base += 256 * K) {
@@ -2171,7 +2199,12 @@ __global__ __launch_bounds__(256) void attn_pv_combine_kernel(AttnArgs a) {
 #pragma unroll
             for (int k = 0; k < K; k++) {
                 const int i = base + (int)threadIdx.x + 256 * k;
-                if (i < total) *(u32x4 *)(stage + 4 * i) = v[k];
+                if (i < total) {
+                    float *at = stage + 4 * (i & (nq - 1)) * cb + (i >> qsh);
+#pragma unroll
+                    for (int e = 0; e < 4; e++)
+                        at[e * cb] = __uint_as_float(e == 0 ? v[k].x : e == 1 ? v[k].y : e == 2 ? v[k].z : v[k].w);
+                }
             }
         }
         __syncthreads();
@@ -2179,19 +2212,23 @@ __global__ __launch_bounds__(256) void attn_pv_combine_kernel(AttnArgs a) {
         for (int k = 0; k < CPT; k++) {
             const int c = threadIdx.x + 256 * k;
             if (c < nc) {
-                int j0 = 0;
-                if (b0 == 0) {
-                    acc[k] = stage[c];
-                    j0 = 1;
-                }
-                for (; j0 + 16 <= cnt; j0 += 16) {  // 16 LDS reads in flight, then adds
-                    float v[16];
-#pragma unroll
-                    for (int u = 0; u < 16; u++) v[u] = stage[(j0 + u) * nc + c];
+                // in block order; 16 are added while the next 16 are read
+                const float *col = stage + c * cb;
+                const int whole = cnt & ~15;
+                float v[16], next[16];
+                if (whole) ld_lds16(col, v);
+                for (int j = 0; j < whole; j += 16) {
+                    ld_lds16(col + min(j + 16, cb - 16), next);
 #pragma unroll
                     for (int u = 0; u < 16; u++) acc[k] += v[u];
+#pragma unroll
+                    for (int u = 0; u < 16; u++) v[u] = next[u];
                 }
-                for (; j0 < cnt; j0++) acc[k] += stage[j0 * nc + c];
+#pragma unroll
+                for (int u = 0; u < 15; u++) v[u] = col[min(whole + u, cnt - 1)];
+#pragma unroll
+                for (int u = 0; u < 15; u++)
+                    if (whole + u < cnt) acc[k] += v[u];
             }
         }
         __syncthreads();
@@ -2496,27 +2533,6 @@ struct SampleSlot {
     float sums[SAMPLE_T];
 };
 static __device__ SampleSlot g_sample_slots[SAMPLE_SLOTS];
-
-// 16 consecutive floats of LDS (16-byte aligned), all requested at once.
-__device__ __forceinline__ void ld_lds16(const float *p, float (&v)[16]) {
-    typedef float f32x4 __attribute__((ext_vector_type(4)));
-    const f32x4 *q = (const f32x4 *)p;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const f32x4 a = q[i];
-        v[4 * i] = a.x;
-        v[4 * i + 1] = a.y;
-        v[4 * i + 2] = a.z;
-        v[4 * i + 3] = a.w;
-    }
-}
-
-__device__ __forceinline__ void st_lds16(float *p, const float (&v)[16]) {
-    typedef float f32x4 __attribute__((ext_vector_type(4)));
-    f32x4 *q = (f32x4 *)p;
-#pragma unroll
-    for (int i = 0; i < 4; i++) q[i] = f32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
-}
 
 // The draw from the SAMPLE_T chunk sums in LDS, by the whole workgroup (every thread calls it after
 // a barrier). Prefix sums of non-negative weights never decrease, so the walk over the chunks is

@@ -421,6 +421,34 @@ def test_attention_one_launch_combine(gpu, oracle, hq, hkv, D, pos, max_seq):
     assert np.array_equal(got, want)
 
 
+@pytest.mark.parametrize("hq,hkv,D", [(8, 1, 64), (2, 1, 128), (4, 1, 128), (1, 1, 256)])
+def test_attention_statistics_chunks(gpu, oracle, hq, hkv, D):
+    """Histories around 1 to 4 chunks of 64 block statistics, and past them, equal the oracle; with
+    scores so far apart that whole blocks weigh nothing, and infinite keys."""
+    import torch
+    ident(f"attention statistics {hq}/{hkv} D{D}")
+    rng = np.random.default_rng(hq * D)
+    max_seq = 16448
+    kc, vc = rand_bf16(rng, (max_seq, hkv * D)), rand_bf16(rng, (max_seq, hkv * D))
+    far = kc.copy()
+    far[4000:9000] = rand_bf16(rng, (5000, hkv * D), 40.0)
+    inf = kc.copy()
+    inf[5000, 3] = 0x7F80
+    att = torch.zeros(gpu.attention_workspace_floats(hq, D, max_seq), device="cuda")
+    scale = float(np.float32(1.0 / np.sqrt(D)))
+    vd = dev(vc)
+    for keys in (kc, far, inf):
+        kd = dev(keys)
+        for pos in (4095, 4096, 8191, 8192, 12287, 12288, 16383, 16384):
+            q = rand_bf16(rng, hq * D)
+            out = dev(np.zeros(hq * D, np.uint16))
+            gpu.attention_forward(out, dev(q), kd, vd, att, hq, hkv, D, dev_i32([pos]), max_seq, scale)
+            want = oracle.attention(q, keys, vc, hq, hkv, D, pos, scale, oracle.GPU_ORDER)
+            got, nan = host(out), np.isnan(bf16_vals(want))
+            assert np.array_equal(got[~nan], want[~nan]), pos
+            assert np.isnan(bf16_vals(got)[nan]).all(), pos
+
+
 FUSED_ATTN_CASES = [(16, 8, 128, 0, 4096), (16, 8, 128, 63, 4096), (16, 8, 128, 64, 4096),
                     (16, 8, 128, 260, 4096), (32, 8, 128, 8192, 8448), (32, 8, 128, 8447, 8448),
                     (8, 8, 128, 100, 512), (8, 1, 128, 130, 512), (2, 2, 64, 301, 512),
