@@ -1038,7 +1038,7 @@ __device__ __forceinline__ void split_attention(KArgs &a, KLayer &L, int pos, in
                 const bool v = b * 64 + lane < n;
                 const float sv = v ? sm.sc[hf][k][w4][lane] : -__builtin_huge_valf();
                 const float m = wave_max<S::SPLIT_STATS_LDS>(sv);
-                const float e = v ? exp_f32(sv - m) : 0.0f;
+                const float e = v ? exp_f32<S::SPLIT_EXP_BRANCHES>(sv - m) : 0.0f;
                 const float ssum = wave_sum<S::SPLIT_STATS_LDS>(e);
                 if (lane == 0) {
                     unsigned long long *st = a.tstat + ((size_t)h * mb + b) * 2;
@@ -1080,7 +1080,7 @@ __device__ __forceinline__ void split_attention(KArgs &a, KLayer &L, int pos, in
 #pragma unroll
             for (int c = 0; c < MAXC; c++) {
                 if (c * 64 >= nb) break;
-                const float cs_ = wave_sum<S::SPLIT_STATS_LDS>(c * 64 + lane < nb ? sv[c] * exp_f32(mv[c] - M) : 0.0f);
+                const float cs_ = wave_sum<S::SPLIT_STATS_LDS>(c * 64 + lane < nb ? sv[c] * exp_f32<S::SPLIT_EXP_BRANCHES>(mv[c] - M) : 0.0f);
                 sum = c == 0 ? cs_ : sum + cs_;
             }
             if (lane == 0) {
@@ -1098,7 +1098,7 @@ __device__ __forceinline__ void split_attention(KArgs &a, KLayer &L, int pos, in
                 if (k >= n_it) break;
                 if (b >= nb) continue;
                 const float sv = sm.sc[hf][k][w4][lane];
-                sm.sc[hf][k][w4][lane] = b * 64 + lane < n ? round_bf(exp_f32(sv - M) / sum) : 0.0f;
+                sm.sc[hf][k][w4][lane] = b * 64 + lane < n ? round_bf(exp_f32<S::SPLIT_EXP_BRANCHES>(sv - M) / sum) : 0.0f;
             }
         }
         __syncthreads();
@@ -1578,7 +1578,7 @@ __global__ __launch_bounds__(THREADS) void step_kernel(StepArgs) {
                 wave_gemv2<NCH, S::B_GU, S::GU_STREAM, SPLIT>(L.w_gate, L.w_up, g0, g1, xb, pf_g, pf_u,
                                          [=](int r, float g, float u) {
                     const bf16 gb = (bf16)f2bf(g), ub = (bf16)f2bf(u);
-                    const float s = round_bf(silu_f32(bf2f(gb)));
+                    const float s = round_bf(silu_f32<SPLIT>(bf2f(gb)));
                     put_tagged_all<I, S::REPLICAS>(hb, r, f2bf(s * bf2f(ub)), tag);
                 });
             }
@@ -1788,6 +1788,9 @@ struct Shape {
     // 4B 441.8-441.9 against 439.0-439.1 with the swizzle (the scores' reduce-scatter through
     // bank_pair_sum in both; alternating runs on one box).
     static constexpr bool SPLIT_STATS_LDS = H <= 2048;
+    // exponentials of the split attention with branches (exp_f32): 4B after 8192 positions 2254 us
+    // per token with, 2323 without; 0.6B 802 with, 770 without
+    static constexpr bool SPLIT_EXP_BRANCHES = H > 2048;
     // q/k/v rows per wave (a prefetched batch; 4B with batches of 2: 575.4-575.9 tokens/s, of 1
     // row 544.7) and
     // where they go. A CU's vector-memory requests complete in order, so a workgroup's poll
