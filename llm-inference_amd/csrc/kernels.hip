@@ -2959,6 +2959,59 @@ __device__ __forceinline__ void block_amax(float &v, int &i, float *lv, int *li)
         for (int k = 1; k < (int)(blockDim.x >> 6); k++) amax_pair(v, i, lv[k], li[k]);
 }
 
+// A row that one workgroup reads in less time than a second launch takes. Each thread sees its elements
+// in ascending order, so a strict comparison keeps the lowest index of its largest value.
+//
+// Bound by its launch and its round trips. One launch here / two launches: 2.8 / 4.4 us at 1000 values,
+// 3.5 / 4.8 at 8192, 4.6 / 4.9 at 24576, 5.2 / 4.9 at 32768.
+constexpr int AMAX_ALONE = 24576, AMAX_ALONE_T = 1024;
+__global__ __launch_bounds__(AMAX_ALONE_T) void argmax_alone_kernel(const bf16 *x, int n, int vec,
+                                                                    int *out) {
+    constexpr int U = 4;  // 16-byte loads of a thread in flight
+    __shared__ float lv[AMAX_ALONE_T / 64];
+    __shared__ int li[AMAX_ALONE_T / 64];
+    const int t = threadIdx.x;
+    float v = -__builtin_huge_valf();
+    int idx = INT_MAX;
+    const auto take = [&](float f, int i) {
+        // -inf counts as a value (lowest index); NaN does not
+        if (f > v || (f == v && i < idx)) {
+            v = f;
+            idx = i;
+        }
+    };
+    int done = 0;
+    if (vec) {
+        const int n_chunks = n / 8;
+        for (int c0 = 0; c0 < n_chunks; c0 += U * AMAX_ALONE_T) {
+            u32x4 ch[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) ch[u] = ld16(x + 8 * min(c0 + u * AMAX_ALONE_T + t, n_chunks - 1));
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                const int c = c0 + u * AMAX_ALONE_T + t;
+                if (c < n_chunks)
+#pragma unroll
+                    for (int e = 0; e < 8; e++) take(elem(ch[u], e), 8 * c + e);
+            }
+        }
+        done = n_chunks * 8;
+    }
+    for (int i = done + t; i < n; i += AMAX_ALONE_T) take(bf2f(x[i]), i);
+    wave_amax(v, idx);
+    if ((t & 63) == 0) {
+        lv[t >> 6] = v;
+        li[t >> 6] = idx;
+    }
+    __syncthreads();
+    if (t < 64) {
+        v = t < AMAX_ALONE_T / 64 ? lv[t] : -__builtin_huge_valf();
+        idx = t < AMAX_ALONE_T / 64 ? li[t] : INT_MAX;
+        wave_amax(v, idx);
+        if (t == 0) *out = idx;
+    }
+}
+
 __global__ __launch_bounds__(256) void argmax_stage1_kernel(const bf16 *x, int n, int vec,
                                                             float *pv, int *pi) {
     __shared__ float lv[4];
@@ -3005,6 +3058,11 @@ static int argmax_groups(int n) {
 
 // Shared by argmax_forward (library buffer) and the step (its own buffer).
 void argmax_launch(int *out, const bf16 *x, int n, float *pv, int *pi, hipStream_t stream) {
+    if (n <= AMAX_ALONE) {
+        argmax_alone_kernel<<<1, AMAX_ALONE_T, 0, stream>>>(x, n, aligned16(x) ? 1 : 0, out);
+        LAUNCH_OK();
+        return;
+    }
     const int groups = argmax_groups(n);
     argmax_stage1_kernel<<<groups, 256, 0, stream>>>(x, n, aligned16(x) ? 1 : 0, pv, pi);
     if (!LAUNCH_OK()) return;

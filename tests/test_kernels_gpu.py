@@ -836,3 +836,23 @@ def test_argmax(gpu, oracle):
     gpu.argmax_forward(out, xd[1:], 1000)
     torch.cuda.synchronize()
     assert int(out.cpu()[0]) == oracle.argmax(x[1:])
+
+
+# around a thread's last chunk and the longest row one workgroup takes (24576)
+@pytest.mark.parametrize("n", [1, 7, 9, 8191, 8192, 8200, 24575, 24576, 24577, 32769])
+def test_argmax_one_and_two_launches(gpu, oracle, n):
+    import torch
+    ident(f"argmax row of {n}")
+    rng = np.random.default_rng(n)
+    out = dev_i32([-5])
+    ties, tail, nan = rand_bf16(rng, n), rand_bf16(rng, n), rand_bf16(rng, n)
+    ties[rng.integers(0, n, 9)] = bf16_bits(np.float32(9.0))
+    tail[n - 1] = bf16_bits(np.float32(9.0)).item()
+    nan[n // 2:] = 0x7FC0
+    lowest = np.full(n, 0xFF80, np.uint16)  # -inf, then NaN
+    lowest[n // 3:] = 0xFFFF
+    for row in (ties, tail, nan, lowest, np.full(n, 0x8000, np.uint16), np.full(n, 0x7FC0, np.uint16)):
+        xd = dev(np.concatenate([row[:1], row]))
+        for x in (dev(row), xd[1:]):
+            gpu.argmax_forward(out, x, n)
+            assert int(out.item()) == oracle.argmax(row)
