@@ -995,13 +995,6 @@ __device__ __forceinline__ void ld_lds16(const float *p, float (&v)[16]) {
     }
 }
 
-__device__ __forceinline__ void st_lds16(float *p, const float (&v)[16]) {
-    typedef float f32x4 __attribute__((ext_vector_type(4)));
-    f32x4 *q = (f32x4 *)p;
-#pragma unroll
-    for (int i = 0; i < 4; i++) q[i] = f32x4{v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]};
-}
-
 constexpr int ATT_B = 64;  // positions per block
 
 struct AttnArgs {
@@ -2508,17 +2501,17 @@ extern "C" void attention_forward_noalloc(bf16 *out, const bf16 *q, const bf16 *
 //
 // Two launches for long rows: sample_kernel, one workgroup, takes the max (a row of 151936 is 300 KB,
 // read from L2); sample_sums_kernel spreads the weights, which are most of the work, over SAMPLE_WGS
-// workgroups, and the last of them to finish adds the chunk sums and draws. Between the two the max
-// and the chunk sums live in one of SAMPLE_SLOTS library-owned slots, taken by the first launch with
-// an atomic exchange and given back by the second, so calls on any streams may overlap; `out` itself
-// carries the slot (as -2 - slot) from one launch to the next. With every slot taken the first
-// launch draws alone, as it does for rows of up to SAMPLE_ALONE.
+// workgroups, and the last of them to finish adds the chunk sums and draws. Between the two the chunk
+// sums live in one of SAMPLE_SLOTS library-owned slots, taken by the first launch with an atomic
+// exchange and given back by the second, so calls on any streams may overlap; `out` itself carries
+// the slot and the max from one launch to the next. With every slot taken the first launch draws
+// alone, as it does for rows of up to SAMPLE_ALONE.
 //
-// Bound by its serial chains, which the order of the additions fixes: 1024 dependent adds for the
-// total (5.5 us measured), about 150 per chunk; the rest is two launches and four round trips to
-// memory. 151936 logits: 119.2 us on one workgroup that also computed every weight, 19.6 us now
-// (6.0 + 13.6); one launch alone now 72 us. The line at SAMPLE_ALONE: alone 9.7 / 11.4 / 16.3 / 22.6
-// us at 4096 / 8192 / 16384 / 32768 logits, spread 15.0-15.5 us at each.
+// Bound by its serial chains, which the order of the additions fixes (1024 dependent adds for the
+// total, about 150 per chunk), two launches and the round trips between them. 151936 logits: 105-119 us
+// on one workgroup, 19.6 us spread over 64, 17.0 us with the chains' LDS reads four deep, the max in the
+// ticket and the slot taken beside the max; 73.7 us on one workgroup now. The line at SAMPLE_ALONE: alone
+// 8.9 / 10.0 / 15.3 / 22.1 us at 4096 / 12288 / 16384 / 32768 logits, spread 13.2-13.5 us at each.
 constexpr int SAMPLE_T = 1024;
 constexpr int SAMPLE_WGS = 64, SAMPLE_ROWS = SAMPLE_T / SAMPLE_WGS;  // chunks per workgroup
 constexpr int SAMPLE_PIECE = 256;  // weights of a chunk staged at a time
@@ -2528,8 +2521,7 @@ constexpr int SAMPLE_ALONE = 12288;  // longest row drawn in one launch
 struct SampleSlot {
     unsigned busy;   // taken by a call
     unsigned done;   // workgroups of the second launch that have published their sums
-    float max;
-    float pad[29];
+    float pad[30];
     float sums[SAMPLE_T];
 };
 static __device__ SampleSlot g_sample_slots[SAMPLE_SLOTS];
@@ -2537,34 +2529,42 @@ static __device__ SampleSlot g_sample_slots[SAMPLE_SLOTS];
 // The draw from the SAMPLE_T chunk sums in LDS, by the whole workgroup (every thread calls it after
 // a barrier). Prefix sums of non-negative weights never decrease, so the walk over the chunks is
 // done on the ends of 64 segments of 16 chunks first (lane s keeps the running sum after segment s:
-// the additions of the total itself), then inside one segment. One wave runs each serial chain.
-__device__ __forceinline__ void sample_draw(int *out, const bf16 *x, int n, float inv_temp, float u,
-                                            float mx, const float *sums, float *piece, float *share) {
+// the additions of the total itself), then inside one segment. One wave runs each serial chain; a
+// dependent addition takes 4.6 clocks and an LDS read some 200, so four reads of 16 sums are in flight.
+__device__ __forceinline__ int sample_draw(const bf16 *x, int n, float inv_temp, float u, float mx,
+                                           const float *sums, float *piece, float *share) {
     const int t = threadIdx.x, lane = t & 63;
     const int chunk = (n + SAMPLE_T - 1) / SAMPLE_T;
+    float v[4][16];
     if (t < 64) {
         // segments that hold chunks with elements (the sums past them are zeros, which add nothing)
         const int segs = ((n + chunk - 1) / chunk + 15) / 16;
-        float total = 0.0f, end = 0.0f, v[16], w[16];
-        ld_lds16(sums, v);
-        for (int s = 0; s < segs; s += 2) {  // two segments a step, each read while the other is added
-            ld_lds16(sums + 16 * min(s + 1, 63), w);
+        float total = 0.0f, end = 0.0f;
 #pragma unroll
-            for (int j = 0; j < 16; j++) total += v[j];
-            end = lane >= s ? total : end;
-            ld_lds16(sums + 16 * min(s + 2, 63), v);
-            if (s + 1 < segs) {
+        for (int q = 0; q < 4; q++) ld_lds16(sums + 16 * q, v[q]);
+        for (int s = 0; s < segs; s += 4) {
 #pragma unroll
-                for (int j = 0; j < 16; j++) total += w[j];
+            for (int q = 0; q < 4; q++) {
+#pragma unroll
+                for (int j = 0; j < 16; j++) total += v[q][j];
+                end = lane >= s + q ? total : end;
+                ld_lds16(sums + 16 * min(s + q + 4, 63), v[q]);
             }
-            end = lane > s ? total : end;
         }
         const float target = u * total;
         const unsigned long long past = __ballot(!(end <= target));
         const int s = past ? __ffsll(past) - 1 : 63;
         float cdf = s > 0 ? __shfl(end, s - 1) : 0.0f;
         int k = 16 * s;
-        while (k < SAMPLE_T - 1 && cdf + sums[k] <= target) cdf += sums[k++];
+        ld_lds16(sums + 16 * s, v[0]);
+        bool on = true;  // never past the segment: its end is past the target, or it is the last
+#pragma unroll
+        for (int j = 0; j < 16; j++) {
+            const float next = cdf + v[0][j];
+            on = on && 16 * s + j < SAMPLE_T - 1 && next <= target;
+            cdf = on ? next : cdf;
+            k += on ? 1 : 0;
+        }
         if (t == 0) {
             share[0] = cdf;
             share[1] = target;
@@ -2584,27 +2584,38 @@ __device__ __forceinline__ void sample_draw(int *out, const bf16 *x, int n, floa
             piece[t] = t < len ? exp_f32((bf2f(x[start + b + t]) - mx) * inv_temp) : 0.0f;
         __syncthreads();
         if (t < 64 && chosen < 0) {
-            // the running sums in place (past the end they add zeros), then the first that passes
-            for (int j = 0; j < len; j += 16) {
-                float v[16];
-                ld_lds16(piece + j, v);
+            // 64 running sums at a time (past the end they add zeros), lane j keeps the j-th; then
+            // the first that passes
 #pragma unroll
-                for (int i = 0; i < 16; i++) v[i] = run = run + v[i];
-                st_lds16(piece + j, v);
-            }
-            for (int j = 0; j < len && chosen < 0; j += 64) {
-                const unsigned long long hit =
-                    __ballot(j + lane < len && cdf + piece[min(j + lane, len - 1)] > target);
-                if (hit) chosen = (int)(start + b + j) + __ffsll(hit) - 1;
+            for (int q = 0; q < 4; q++) ld_lds16(piece + 16 * q, v[q]);
+            for (int j0 = 0; j0 < len && chosen < 0; j0 += 64) {
+                float mine = 0.0f;
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+#pragma unroll
+                    for (int j = 0; j < 16; j++) {
+                        run += v[q][j];
+                        mine = lane >= 16 * q + j ? run : mine;
+                    }
+                    ld_lds16(piece + min(j0 + 64 + 16 * q, SAMPLE_PIECE - 16), v[q]);
+                }
+                const unsigned long long hit = __ballot(j0 + lane < len && cdf + mine > target);
+                if (hit) chosen = (int)(start + b + j0) + __ffsll(hit) - 1;
             }
         }
         __syncthreads();
     }
-    if (t == 0) *out = chosen;
+    return chosen;  // in the first wave
+}
+
+// What the first launch leaves in *out for the second: bit 31, the slot, and the row's max, which is
+// one of its bf16 values. (No drawn token looks like it: indexes have bit 31 clear, -1 has no slot.)
+__device__ __forceinline__ uint32_t sample_ticket(int slot, float mx) {
+    return 0x80000000u | (uint32_t)slot << 16 | __float_as_uint(mx) >> 16;
 }
 
 // The max of the row, then either the slot for sample_sums_kernel (spread != 0) or the whole draw.
-// vec: x is 16-byte aligned.
+// The last wave takes the slot before it reads its part of the row. vec: x is 16-byte aligned.
 __global__ __launch_bounds__(SAMPLE_T) void sample_kernel(int *out, const bf16 *x, int n,
                                                           float inv_temp, float u, int vec,
                                                           int spread) {
@@ -2614,6 +2625,30 @@ __global__ __launch_bounds__(SAMPLE_T) void sample_kernel(int *out, const bf16 *
     __shared__ float share[3];
     __shared__ int s_slot;
     const int t = threadIdx.x;
+    if (spread && wave_id() == SAMPLE_T / 64 - 1) {
+        // lanes 0 .. SAMPLE_SLOTS - 1 look at one slot each, the lowest free one is taken
+        const int lane = t & 63;
+        int slot = -1;
+        const bool free = lane < SAMPLE_SLOTS &&
+                          __hip_atomic_load(gptr(&g_sample_slots[lane & (SAMPLE_SLOTS - 1)].busy),
+                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
+        unsigned long long left = __ballot(free);
+        while (left && slot < 0) {
+            const int s = __ffsll(left) - 1;
+            left &= left - 1;
+            unsigned was = 1;
+            if (lane == 0)
+                was = __hip_atomic_exchange(gptr(&g_sample_slots[s].busy), 1u, __ATOMIC_RELAXED,
+                                            __HIP_MEMORY_SCOPE_AGENT);
+            if (__builtin_amdgcn_readfirstlane(was) == 0) slot = s;
+        }
+        if (lane == 0) {
+            s_slot = slot;
+            if (slot >= 0)
+                __hip_atomic_store(gptr(&g_sample_slots[slot].done), 0u, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
     float m = -__builtin_huge_valf();
     int done = 0;
     if (vec) {
@@ -2638,36 +2673,9 @@ __global__ __launch_bounds__(SAMPLE_T) void sample_kernel(int *out, const bf16 *
     float mx = wmax[0];
 #pragma unroll
     for (int w = 1; w < SAMPLE_T / 64; w++) mx = fmaxf(mx, wmax[w]);  // max: any order
-    if (spread) {
-        if (t < 64) {
-            // lanes 0 .. SAMPLE_SLOTS - 1 look at one slot each, the lowest free one is taken
-            int slot = -1;
-            bool free = t < SAMPLE_SLOTS &&
-                        __hip_atomic_load(gptr(&g_sample_slots[t & (SAMPLE_SLOTS - 1)].busy),
-                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
-            unsigned long long left = __ballot(free);
-            while (left && slot < 0) {
-                const int s = __ffsll(left) - 1;
-                left &= left - 1;
-                unsigned was = 1;
-                if (t == 0)
-                    was = __hip_atomic_exchange(gptr(&g_sample_slots[s].busy), 1u, __ATOMIC_ACQUIRE,
-                                                __HIP_MEMORY_SCOPE_AGENT);
-                if (__builtin_amdgcn_readfirstlane(was) == 0) slot = s;
-            }
-            if (t == 0) {
-                s_slot = slot;
-                if (slot >= 0) {
-                    __hip_atomic_store(gptr(&g_sample_slots[slot].max), mx, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-                    __hip_atomic_store(gptr(&g_sample_slots[slot].done), 0u, __ATOMIC_RELAXED,
-                                       __HIP_MEMORY_SCOPE_AGENT);
-                    *out = -2 - slot;
-                }
-            }
-        }
-        __syncthreads();
-        if (s_slot >= 0) return;
+    if (spread && s_slot >= 0) {
+        if (t == 0) *out = (int)sample_ticket(s_slot, mx);
+        return;
     }
     const int chunk = (n + SAMPLE_T - 1) / SAMPLE_T;
     const long long start = (long long)t * chunk, end = min(start + chunk, (long long)n);
@@ -2675,7 +2683,8 @@ __global__ __launch_bounds__(SAMPLE_T) void sample_kernel(int *out, const bf16 *
     for (long long i = start; i < end; i++) acc += exp_f32((bf2f(x[i]) - mx) * inv_temp);
     sums[t] = acc;
     __syncthreads();
-    sample_draw(out, x, n, inv_temp, u, mx, sums, piece, share);
+    const int chosen = sample_draw(x, n, inv_temp, u, mx, sums, piece, share);
+    if (t == 0) *out = chosen;
 }
 
 // Workgroup w: the sums of chunks [w SAMPLE_ROWS, (w + 1) SAMPLE_ROWS). All threads compute the
@@ -2703,11 +2712,11 @@ __global__ __launch_bounds__(256) void sample_sums_kernel(int *out, const bf16 *
                 v[r][j] = x[min(at, (long long)n - 1)];
             }
     };
-    request(0);  // before the slot's two dependent reads
-    const int slot = -2 - *out;
-    if (slot < 0 || slot >= SAMPLE_SLOTS) return;  // the first launch has drawn (or *out is no slot)
-    SampleSlot &sl = g_sample_slots[slot];
-    const float mx = __hip_atomic_load(gptr(&sl.max), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    request(0);  // before the wait for the ticket
+    const uint32_t ticket = (uint32_t)*out;
+    if (!(ticket >> 31) || (ticket >> 16 & 0x7fff) >= SAMPLE_SLOTS) return;  // the first launch has drawn
+    SampleSlot &sl = g_sample_slots[ticket >> 16 & 0x7fff];
+    const float mx = __uint_as_float(ticket << 16);
     float acc = 0.0f;
     for (int b = 0; b < chunk; b += P) {
         const int len = min(P, chunk - b);
@@ -2725,22 +2734,35 @@ __global__ __launch_bounds__(256) void sample_sums_kernel(int *out, const bf16 *
             const long long at = (long long)(k0 + t) * chunk + b;
             const int have = at >= n ? 0 : (int)min((long long)len, n - at);
             const float *row = stage + t * (P + 1);
+            float e[2][16];
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int i = 0; i < 16; i++) e[h][i] = row[16 * h + i];
             int j = 0;
-            for (; j + 16 <= have; j += 16) {
-                float e[16];
+            for (; j + 32 <= have; j += 32)
 #pragma unroll
-                for (int i = 0; i < 16; i++) e[i] = row[j + i];
+                for (int h = 0; h < 2; h++) {
 #pragma unroll
-                for (int i = 0; i < 16; i++) acc += e[i];
-            }
-            for (; j < have; j++) acc += row[j];
+                    for (int i = 0; i < 16; i++) acc += e[h][i];
+#pragma unroll
+                    for (int i = 0; i < 16; i++) e[h][i] = row[min(j + 32 + 16 * h, P - 16) + i];
+                }
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+#pragma unroll
+                for (int i = 0; i < 16; i++)
+                    if (j + 16 * h + i < have) acc += e[h][i];
         }
         __syncthreads();
     }
     if (t < R)
         __hip_atomic_store(gptr(&sl.sums[k0 + t]), acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (t == 0)  // the same wave's stores come before its arrival
-        s_last = __hip_atomic_fetch_add(gptr(&sl.done), 1u, __ATOMIC_ACQ_REL,
+    // The sums are written through to the level all XCDs share, by this wave alone: once they are
+    // acknowledged there, the arrival needs no release of its own (which writes back the whole L2).
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (t == 0)
+        s_last = __hip_atomic_fetch_add(gptr(&sl.done), 1u, __ATOMIC_RELAXED,
                                         __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
     __syncthreads();
     if (!s_last) return;
@@ -2753,9 +2775,10 @@ __global__ __launch_bounds__(256) void sample_sums_kernel(int *out, const bf16 *
 #pragma unroll
     for (int i = 0; i < SAMPLE_T / 256; i++) sums[t + 256 * i] = got[i];
     __syncthreads();
-    if (t == 0)  // nothing reads the slot any more
-        __hip_atomic_store(gptr(&sl.busy), 0u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-    sample_draw(out, x, n, inv_temp, u, mx, sums, piece, share);
+    if (t == 0)  // every sum has been read
+        __hip_atomic_store(gptr(&sl.busy), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int chosen = sample_draw(x, n, inv_temp, u, mx, sums, piece, share);
+    if (t == 0) *out = chosen;
 }
 
 extern "C" void sample_forward(int *out, const bf16 *x, int n, float inv_temp, float u,
