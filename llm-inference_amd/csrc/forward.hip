@@ -23,6 +23,13 @@ static bool dmalloc(void **p, size_t bytes) {
     return HIP_OK(hipMemset(*p, 0, bytes));
 }
 
+// The words through which a step's token and error flag reach the host: pinned, written by a kernel, so
+// that reading them costs no copy.
+static bool alloc_mail(RunState *s) {
+    return HIP_OK(hipHostMalloc((void **)&s->mail, 64, hipHostMallocMapped)) &&
+           HIP_OK(hipHostGetDevicePointer((void **)&s->mail_dev, s->mail, 0));
+}
+
 extern "C" void alloc_run_state_seq(RunState *s, const Config *cfg, int max_seq) {
     memset(s, 0, sizeof *s);
     if (max_seq <= 0) {
@@ -47,6 +54,7 @@ extern "C" void alloc_run_state_seq(RunState *s, const Config *cfg, int max_seq)
               dmalloc((void **)&s->logits, (size_t)cfg->vocab_size * 2) &&
               dmalloc((void **)&s->next_token, 4) && dmalloc((void **)&s->pos, 4) &&
               dmalloc(&s->argmax_partials, (size_t)argmax_partial_count() * 8) &&
+              dmalloc(&s->sample_slot, sample_slot_bytes()) && alloc_mail(s) &&
               dmalloc((void **)&s->pos_base, 4) && dmalloc((void **)&s->error_flag, 4) &&
               dmalloc(&s->step_ws, step_workspace_bytes(cfg, max_seq)) &&
               dmalloc((void **)&s->rope_table, (size_t)cfg->head_dim * 4);
@@ -66,9 +74,10 @@ extern "C" void free_run_state(RunState *s) {
                     s->att, s->key_cache, s->value_cache, s->hb, s->tap1, s->tap2,
                     s->logits, s->next_token, s->pos, s->argmax_partials, s->token_out,
                     s->pos_base, s->error_flag, s->step_ws, s->layers_dev,
-                    s->attn_one_pass_ws, s->rope_table};
+                    s->attn_one_pass_ws, s->rope_table, s->sample_slot};
     for (void *b : bufs)
         if (b) HIP_OK(hipFree(b));
+    if (s->mail) HIP_OK(hipHostFree(s->mail));
     if (s->graph) HIP_OK(hipGraphExecDestroy(s->graph));
     if (s->loop_graph) HIP_OK(hipGraphExecDestroy(s->loop_graph));
     if (s->stream) HIP_OK(hipStreamDestroy(s->stream));
@@ -420,33 +429,56 @@ extern "C" void forward(const Config *cfg, const Weights *w, RunState *s, int to
     }
 }
 
-// src/forward.cu:229-236
-// src/forward.cu:238-251: a token drawn from softmax(logits / temperature) at the coin; the
-// argmax a persistent step left in next_token is overwritten.
-extern "C" int sample_temperature(const Config *cfg, RunState *s, float temperature, float coin) {
-    const float inv_temp = 1.0f / temperature;
-    sample_forward(s->next_token, s->logits, cfg->vocab_size, inv_temp, coin, s->stream);
-    s->next_token_valid = 0;
-    int token = -1;
-    if (!HIP_OK(hipMemcpyAsync(&token, s->next_token, 4, hipMemcpyDeviceToHost, s->stream)))
-        return -1;
-    if (!HIP_OK(hipStreamSynchronize(s->stream))) return -1;
-    if (!check_step_error(cfg, s)) return -1;
-    if (token < 0) {
-        llm_fail("sampling found no token (coin %g)", (double)coin);
-        return -1;
+// Token and error flag to the host.
+__global__ void mail_kernel(int *mail, const int *next_token, const int *err) {
+    if (threadIdx.x == 0) {
+        mail[0] = *next_token;
+        mail[1] = *err;
     }
-    return token;
 }
 
+// Waits for the stream, whose last kernel has written the mail, and returns the token, or -1 after an
+// error.
+static int read_mail(const Config *cfg, RunState *s) {
+    if (!HIP_OK(hipStreamSynchronize(s->stream))) return -1;
+    const volatile int *mail = s->mail;
+    if (mail[1] != 0 && !check_step_error(cfg, s)) return -1;
+    return mail[0];
+}
+
+static bool send_mail(RunState *s) {
+    mail_kernel<<<1, 64, 0, s->stream>>>(s->mail_dev, s->next_token, s->error_flag);
+    return LAUNCH_OK();
+}
+
+// src/forward.cu:238-251: a token drawn from softmax(logits / temperature) at the coin; the
+// argmax a persistent step left in next_token is overwritten (it tells the draw the largest logit).
+//
+// The token and the error flag used to be copied to pageable host memory one after the other, each with
+// its own wait, after a launch that took the row's max. A sampled token, Qwen3-1.7B after 3000
+// positions: 1181 -> 1144 us; 0.6B after 8192 836 -> 808; 12 layers of 512 on the hipGraph 171 -> 151.
+extern "C" int sample_temperature(const Config *cfg, RunState *s, float temperature, float coin) {
+    const float inv_temp = 1.0f / temperature;
+    if (s->next_token_valid) {
+        s->next_token_valid = 0;
+        if (!sample_known_max(s->next_token, s->logits, cfg->vocab_size, inv_temp, coin,
+                              s->sample_slot, s->mail_dev, s->error_flag, s->stream))
+            return -1;
+    } else {
+        sample_forward(s->next_token, s->logits, cfg->vocab_size, inv_temp, coin, s->stream);
+        if (!send_mail(s)) return -1;
+    }
+    const int token = read_mail(cfg, s);
+    if (token < 0 && !llm_has_error())
+        llm_fail("sampling found no token (coin %g)", (double)coin);
+    return token < 0 ? -1 : token;
+}
+
+// src/forward.cu:229-236
 extern "C" int sample_argmax(const Config *cfg, RunState *s) {
     if (!s->next_token_valid) argmax_into_next(cfg, s);  // the persistent step already did it
-    int token = -1;
-    if (!HIP_OK(hipMemcpyAsync(&token, s->next_token, 4, hipMemcpyDeviceToHost, s->stream)))
-        return -1;
-    if (!HIP_OK(hipStreamSynchronize(s->stream))) return -1;
-    if (!check_step_error(cfg, s)) return -1;
-    return token;
+    if (!send_mail(s)) return -1;
+    return read_mail(cfg, s);
 }
 
 // token_out holds at least n tokens (a larger buffer drops the loop graph, which captured the

@@ -2519,7 +2519,7 @@ constexpr int SAMPLE_SLOTS = 16;
 constexpr int SAMPLE_ALONE = 12288;  // longest row drawn in one launch
 
 struct SampleSlot {
-    unsigned busy;   // taken by a call
+    unsigned busy;   // taken by a call (of the library's slots)
     unsigned done;   // workgroups of the second launch that have published their sums
     float pad[30];
     float sums[SAMPLE_T];
@@ -2687,11 +2687,21 @@ __global__ __launch_bounds__(SAMPLE_T) void sample_kernel(int *out, const bf16 *
     if (t == 0) *out = chosen;
 }
 
+// A call that knows where the row's max is (a decode step that has its argmax) and has a slot of its
+// own needs no first launch: *out holds the index of the max, and the drawn token is also handed to the
+// host, with the step's error flag, in the two pinned words at mail.
+struct SampleStep {
+    SampleSlot *slot;  // NULL: the slot and the max are in the ticket
+    int *mail;
+    const int *err;
+};
+
 // Workgroup w: the sums of chunks [w SAMPLE_ROWS, (w + 1) SAMPLE_ROWS). All threads compute the
 // weights of a piece of each chunk into LDS (four chunks per wave, one lane per weight), then lane r
 // of the first wave adds chunk r's in order. The workgroup that publishes last draws.
 __global__ __launch_bounds__(256) void sample_sums_kernel(int *out, const bf16 *x, int n,
-                                                          float inv_temp, float u) {
+                                                          float inv_temp, float u,
+                                                          SampleStep step) {
     constexpr int R = SAMPLE_ROWS, P = SAMPLE_PIECE, RW = R / 4;
     __shared__ __align__(16) float stage[R * (P + 1)];  // padded rows: lanes 0..R-1 read one column
     __shared__ float share[3];
@@ -2714,9 +2724,17 @@ __global__ __launch_bounds__(256) void sample_sums_kernel(int *out, const bf16 *
     };
     request(0);  // before the wait for the ticket
     const uint32_t ticket = (uint32_t)*out;
-    if (!(ticket >> 31) || (ticket >> 16 & 0x7fff) >= SAMPLE_SLOTS) return;  // the first launch has drawn
-    SampleSlot &sl = g_sample_slots[ticket >> 16 & 0x7fff];
-    const float mx = __uint_as_float(ticket << 16);
+    SampleSlot *slot = step.slot;
+    float mx;
+    if (slot) {  // an index past the row (no element is a number): the max of no numbers
+        mx = ticket < (uint32_t)n ? bf2f(x[ticket]) : -__builtin_huge_valf();
+    } else {
+        // not a ticket: the first launch has drawn
+        if (!(ticket >> 31) || (ticket >> 16 & 0x7fff) >= SAMPLE_SLOTS) return;
+        slot = &g_sample_slots[ticket >> 16 & 0x7fff];
+        mx = __uint_as_float(ticket << 16);
+    }
+    SampleSlot &sl = *slot;
     float acc = 0.0f;
     for (int b = 0; b < chunk; b += P) {
         const int len = min(P, chunk - b);
@@ -2775,10 +2793,20 @@ __global__ __launch_bounds__(256) void sample_sums_kernel(int *out, const bf16 *
 #pragma unroll
     for (int i = 0; i < SAMPLE_T / 256; i++) sums[t + 256 * i] = got[i];
     __syncthreads();
-    if (t == 0)  // every sum has been read
-        __hip_atomic_store(gptr(&sl.busy), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (t == 0) {  // every sum has been read
+        if (step.slot)
+            __hip_atomic_store(gptr(&sl.done), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        else
+            __hip_atomic_store(gptr(&sl.busy), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     const int chosen = sample_draw(x, n, inv_temp, u, mx, sums, piece, share);
-    if (t == 0) *out = chosen;
+    if (t == 0) {
+        *out = chosen;
+        if (step.mail) {
+            step.mail[0] = chosen;
+            step.mail[1] = *step.err;
+        }
+    }
 }
 
 extern "C" void sample_forward(int *out, const bf16 *x, int n, float inv_temp, float u,
@@ -2790,8 +2818,17 @@ extern "C" void sample_forward(int *out, const bf16 *x, int n, float inv_temp, f
     const int spread = n > SAMPLE_ALONE;
     sample_kernel<<<1, SAMPLE_T, 0, stream>>>(out, x, n, inv_temp, u, aligned16(x) ? 1 : 0, spread);
     if (!LAUNCH_OK() || !spread) return;
-    sample_sums_kernel<<<SAMPLE_WGS, 256, 0, stream>>>(out, x, n, inv_temp, u);
+    sample_sums_kernel<<<SAMPLE_WGS, 256, 0, stream>>>(out, x, n, inv_temp, u, SampleStep{});
     LAUNCH_OK();
+}
+
+size_t sample_slot_bytes() { return sizeof(SampleSlot); }
+
+bool sample_known_max(int *out, const bf16 *x, int n, float inv_temp, float u, void *slot, int *mail,
+                      const int *err, hipStream_t stream) {
+    sample_sums_kernel<<<SAMPLE_WGS, 256, 0, stream>>>(
+        out, x, n, inv_temp, u, SampleStep{(SampleSlot *)slot, mail, err});
+    return LAUNCH_OK();
 }
 
 // ------------------------------------------------------------------------------------------

@@ -54,7 +54,7 @@ class RunState(ctypes.Structure):
                 ("next_token_valid", _i), ("step_trace", ctypes.POINTER(ctypes.c_longlong)),
                 ("attn_mode", _i), ("attn_one_pass_ws", _vp),
                 ("rope_table", ctypes.POINTER(ctypes.c_float)), ("step_switch_pos", _i),
-                ("step_split_blocks", _i)]
+                ("step_split_blocks", _i), ("sample_slot", _vp), ("mail", _vp), ("mail_dev", _vp)]
 
 
 STEP_MODES = {"auto": 0, "graph": 1, "persistent": 2}

@@ -157,6 +157,33 @@ def test_sample_temperature_step(small_model, oracle):
         assert dec.sample_temperature(temp, coin) == oracle.sample(lg, np.float32(1.0 / temp), coin)
 
 
+@pytest.mark.parametrize("mode", ["persistent", "graph"])
+def test_draws_and_argmax_follow_each_step(gpu, oracle, mode):
+    """One draw after each step (the step kernel's argmax gives the draw its max) and, in between, a
+    second draw, an argmax and a draw after it from the same logits: each as the oracle's."""
+    from llm_inference_amd import model
+    ident(f"draws after each {mode} step")
+    cfg = model.make_config(512, 1024, 2, 8, 4, vocab_size=4099, max_seq_len=64)
+    dec = model.Decoder(cfg, ("synth", 11, 0.05, 0.1))
+    dec.capture_graph(mode)
+    tok = 7
+    for pos, (temp, coin) in enumerate([(1.0, 0.3), (0.25, 0.999999), (4.0, 0.0), (0.7, 0.5), (1.3, 0.9)]):
+        dec.forward(tok, pos)
+        logits = dec.logits()
+        want = [oracle.sample(logits, np.float32(1.0 / temp), c) for c in (coin, 0.6)]
+        if pos != 3:
+            tok = dec.sample_temperature(temp, coin)
+            assert tok == want[0]
+        assert dec.sample_temperature(temp, 0.6) == want[1]
+        if pos >= 2:
+            dec.forward(tok, pos)
+            best = oracle.argmax(dec.logits())
+            assert dec.sample_argmax() == best and dec.sample_argmax() == best
+            assert dec.sample_temperature(temp, coin) == oracle.sample(
+                dec.logits(), np.float32(1.0 / temp), coin)
+    dec.close()
+
+
 # ref/compare.py:13-18: worst-row relative L2 error per dumped tensor (embed and layer 0 held
 # tighter), and the near-tie rule for the logits' argmax
 DUMP_TOL_FIRST, DUMP_TOL = 0.02, 0.15
