@@ -1021,7 +1021,7 @@ constexpr uint32_t ATT_UNWRITTEN = 0xffffffffu;
 template <int D, int REP>
 __device__ __forceinline__ void mark_partials(const AttnArgs &a, int b, int g) {
     constexpr int Q = D / 4;  // 16-byte stores per head
-    for (int i = threadIdx.x; i < REP * Q; i += 256)
+    for (int i = tid_x(); i < REP * Q; i += 256)
         st16(a.partial + ((size_t)(g * REP + i / Q) * a.max_blocks + b) * D + 4 * (i % Q),
              u32x4{ATT_UNWRITTEN, ATT_UNWRITTEN, ATT_UNWRITTEN, ATT_UNWRITTEN});
 }
@@ -1038,6 +1038,23 @@ static size_t attention_partial_offset(int n_heads, int max_seq) {
 extern "C" size_t attention_workspace_floats(int n_heads, int head_dim, int max_seq) {
     const size_t mb = ceil_div((size_t)max_seq, ATT_B);
     return attention_partial_offset(n_heads, max_seq) + (size_t)n_heads * mb * head_dim;
+}
+
+// This lane's chunks (16 bytes at 8 L) of the rows first, first + PPW, ... of block b of a cache, kv
+// head g: the block's rows below `rows` as one buffer, so that those at or past it read zeros with no
+// branch around the loads.
+template <int D, int ITERS>
+__device__ __forceinline__ void request_rows(const bf16 *cache, int kv_dim, int b, int g, int rows,
+                                             int first, int L, u32x4 (&out)[ITERS]) {
+    constexpr int PPW = 512 / D;  // positions of a wave's load
+    const int have = min(ATT_B, rows - b * ATT_B);
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(cache + (size_t)b * ATT_B * kv_dim + g * D), (short)0,
+        have <= 0 ? 0 : ((have - 1) * kv_dim + D) * 2, BUFFER_FLAGS);
+#pragma unroll
+    for (int it = 0; it < ITERS; it++)
+        out[it] = __builtin_amdgcn_raw_buffer_load_b128(
+            rs, ((first + it * PPW) * kv_dim + 8 * L) * 2, 0, BUFFER_NT);
 }
 
 // Pass 1, per (block of 64 positions, kv head): scores of the REP query heads sharing the kv
@@ -1059,11 +1076,7 @@ __global__ __launch_bounds__(256) void attn_scores_kernel(AttnArgs a) {
 #pragma unroll
         for (int r = 0; r < REP; r++) qv[r] = ld16(a.q + (size_t)(g * REP + r) * D + 8 * L);
         u32x4 kv[ITERS];
-#pragma unroll
-        for (int it = 0; it < ITERS; it++) {
-            const int t = b * ATT_B + w * PER_WAVE + it * PPW + G;
-            kv[it] = t < n ? ld16_nt(a.kc + (size_t)t * kv_dim + g * D + 8 * L) : u32x4{0, 0, 0, 0};
-        }
+        request_rows<D, ITERS>(a.kc, kv_dim, b, g, n, w * PER_WAVE + G, L, kv);
         // the ITERS * REP dot products of a lane, reduced over the LP lanes of its position group
         // LP at a time by reduce-scatter (each total bit-identical to group_sum<LP>): lane L of a
         // slice ends with product scatter_row(L) of that slice
@@ -1150,8 +1163,8 @@ bool rope_table_launch(float *table, const int *d_pos, int head_dim, float theta
     return LAUNCH_OK();
 }
 
-// The rope inputs of one wave (the raw head rows and norm weights), requested before the key
-// rows so that they are not behind them (loads complete in order), and the RoPE table.
+// The rope inputs of one wave of the one-pass kernel (the raw head rows and norm weights, requested
+// before the key rows so that they are not behind them: loads complete in order) and its RoPE table.
 template <int D>
 struct RopeIn {
     u32x4 xa, xb, wa, wb;
@@ -1182,20 +1195,31 @@ __device__ __forceinline__ LaneFreq<D> lane_freq(const float (&table)[128]) {
     return out;
 }
 
+// The rope inputs of one wave: the raw head rows and norm weights, and the lane's part of the RoPE
+// table: TABLE: the entries of its rotation pairs 8 L .. 8 L + 7, read from the step's table; else the
+// frequencies of the entries it computes, inv_freq[lane + 64 m].
+template <int D, bool TABLE>
+struct ScoresRopeIn {
+    u32x4 xa, xb, wa, wb;
+    u32x4 cs[TABLE ? 2 : 1], sn[TABLE ? 2 : 1];
+    float freq[RopeShape<D>::NJ];
+    __device__ float operator[](int j) const { return freq[j >> 6]; }  // j = lane + 64 m
+};
+
 // Waves 0 .. QWAVES-1 take the kv head's REP query heads (HPW per wave, the qk_norm_rope_kernel
-// lane layout); wave QWAVES the key head when `key`. Returns whether this wave has rope work.
-template <int D, int REP>
-__device__ __forceinline__ bool rope_request(const AttnRopeArgs &r, int g, int pos, bool key,
-                                             RopeIn<D> &in) {
+// lane layout); wave QWAVES the key head. Every wave issues the requests, the others' read nothing
+// (empty buffers), so no branch joins before the key rows. Returns whether the wave has heads (wave
+// QWAVES: if the item holds the position).
+template <int D, int REP, bool TABLE>
+__device__ __forceinline__ bool rope_request(const AttnRopeArgs &r, int g, ScoresRopeIn<D, TABLE> &in) {
     constexpr int LH = D / 16, HPW = 64 / LH, HALF = D / 2;
     constexpr int QWAVES = (REP + HPW - 1) / HPW;
     static_assert(QWAVES < 4 && HPW >= 2, "rope waves");
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    if (w > QWAVES || (w == QWAVES && !key)) return false;
-    const int lane = threadIdx.x & 63, hg = lane / LH, L = lane % LH;
-    const bool is_k = w == QWAVES;
+    const int w = wave_id();
+    const int lane = tid_x() & 63, hg = lane / LH, L = lane % LH;
+    const bool is_k = w == QWAVES, any = w <= QWAVES;
     const int hl0 = is_k ? 0 : w * HPW;
-    const int n_h = is_k ? 1 : min(HPW, REP - hl0);
+    const int n_h = !any ? 0 : is_k ? 1 : min(HPW, REP - hl0);
     const bf16 *src = is_k ? r.k + (size_t)g * D : r.at.q + ((size_t)g * REP + hl0) * D;
     // the wave's heads as one wave-uniform buffer: loads past the last head read zeros
     const __amdgpu_buffer_rsrc_t xr =
@@ -1203,27 +1227,61 @@ __device__ __forceinline__ bool rope_request(const AttnRopeArgs &r, int g, int p
     const int oa = hg * D * 2 + 16 * L, ob = oa + 2 * HALF;
     in.xa = __builtin_amdgcn_raw_buffer_load_b128(xr, oa, 0, 0);
     in.xb = __builtin_amdgcn_raw_buffer_load_b128(xr, ob, 0, 0);
-    const bf16 *nw = is_k ? r.kn : r.qn;
-    in.wa = ld16(nw + 8 * L);
-    in.wb = ld16(nw + HALF + 8 * L);
-    return true;
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+        (void *)(is_k ? r.kn : r.qn), (short)0, any ? D * 2 : 0, BUFFER_FLAGS);
+    in.wa = __builtin_amdgcn_raw_buffer_load_b128(wr, 16 * L, 0, 0);
+    in.wb = __builtin_amdgcn_raw_buffer_load_b128(wr, 16 * L + 2 * HALF, 0, 0);
+    if constexpr (TABLE) {
+        const __amdgpu_buffer_rsrc_t tr = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)r.table, (short)0, any ? 2 * HALF * 4 : 0, BUFFER_FLAGS);
+#pragma unroll
+        for (int i = 0; i < 2; i++) {
+            in.cs[i] = __builtin_amdgcn_raw_buffer_load_b128(tr, 32 * L + 16 * i, 0, 0);
+            in.sn[i] = __builtin_amdgcn_raw_buffer_load_b128(tr, HALF * 4 + 32 * L + 16 * i, 0, 0);
+        }
+    } else {
+        // in the argument segment itself (the address of the by-value argument would be a copy's)
+        const char *args = (const char *)__builtin_amdgcn_kernarg_segment_ptr();
+        const __amdgpu_buffer_rsrc_t fr = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(args + offsetof(AttnRopeArgs, inv_freq)), (short)0, any ? HALF * 4 : 0,
+            BUFFER_FLAGS);
+#pragma unroll
+        for (int m = 0; m < RopeShape<D>::NJ; m++)
+            in.freq[m] = __uint_as_float(
+                __builtin_amdgcn_raw_buffer_load_b32(fr, 4 * (lane + 64 * m), 0, 0));
+    }
+    return any;
 }
 
 // QK-norm + RoPE of the requested heads into q_out / k_out (LDS); the key wave also writes k'
 // and (its next group of lanes) the value row into the caches' row pos.
-template <int D, int REP>
+template <int D, int REP, bool TABLE>
 __device__ __forceinline__ void rope_finish(const AttnRopeArgs &r, int g, int pos,
-                                            const RopeIn<D> &in, u32x4 *q_out, u32x4 *k_out) {
+                                            const ScoresRopeIn<D, TABLE> &in, u32x4 *q_out,
+                                            u32x4 *k_out) {
     constexpr int LH = D / 16, HPW = 64 / LH, HALF = D / 2;
     constexpr int QWAVES = (REP + HPW - 1) / HPW;
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63, hg = lane / LH, L = lane % LH;
+    const int w = wave_id();
+    const int lane = tid_x() & 63, hg = lane / LH, L = lane % LH;
     const bool is_k = w == QWAVES;
     const int hl0 = is_k ? 0 : w * HPW;
     const int n_h = is_k ? 1 : min(HPW, REP - hl0);
     const size_t kv_dim = (size_t)r.at.n_kv_heads * D;
     u32x4 ya, yb, va, vb;
-    norm_rope<D>(in.xa, in.xb, in.wa, in.wb, r.eps, in.cs, in.sn, L, ya, yb, va, vb);
+    float c[8], s[8];
+    if constexpr (TABLE) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const u32x4 &cw = in.cs[e / 4], &sw = in.sn[e / 4];
+            c[e] = __uint_as_float(e % 4 == 0 ? cw.x : e % 4 == 1 ? cw.y : e % 4 == 2 ? cw.z : cw.w);
+            s[e] = __uint_as_float(e % 4 == 0 ? sw.x : e % 4 == 1 ? sw.y : e % 4 == 2 ? sw.z : sw.w);
+        }
+    } else {
+        float cs[RopeShape<D>::NJ], sn[RopeShape<D>::NJ];
+        rope_table<D>(pos, in, cs, sn);
+        rope_fetch<D>(cs, sn, L, c, s);
+    }
+    norm_rope_with<D>(in.xa, in.xb, in.wa, in.wb, r.eps, c, s, ya, yb, va, vb);
     if (hg < n_h) {
         u32x4 *dst = is_k ? k_out : q_out + (hl0 + hg) * (D / 8);
         dst[L] = va;
@@ -1241,56 +1299,46 @@ __device__ __forceinline__ void rope_finish(const AttnRopeArgs &r, int g, int po
     }
 }
 
-// TABLE: the RoPE table comes from r.table (a small load issued with the rope inputs) instead of
-// being computed in double precision by every item. The kernel then fits 96 registers without
-// spills for D <= 128 and REP <= 4 (five workgroups per CU instead of four: Qwen3-4B's 1056 items
-// at 8448 positions are resident in one wave of 1280 slots) and its items' rope chain is shorter.
+// TABLE: the RoPE table comes from r.table, each lane its own entries, instead of being computed in
+// double precision by every item and fetched from the lanes that computed them. The kernel then fits 96
+// registers without spills for D <= 128 and REP <= 4 (five workgroups per CU instead of four: Qwen3-4B's
+// 1056 items at 8448 positions are resident in one wave of 1280 slots) and its items' rope chain is
+// shorter.
+//
+// Bound by its chain (the heads' norm and rotation, the products, the exponentials) beside the key
+// stream. With the table's entries shuffled in 16 steps, a branch around each key row's load and lane
+// values held over the item loop, the Qwen3-1.7B hipGraph step took 1189 us after 5000 positions and
+// 1287 after 8300, 4B 2099 after 4300 and 2249 after 8200; now 1153, 1246, 2070 and 2200. (Requesting
+// the rope inputs, or the next pass's statistics, before the position is known changed nothing.)
 template <int D, int REP, bool TABLE>
 __global__ __launch_bounds__(256)
 __attribute__((amdgpu_waves_per_eu(TABLE && D <= 128 && REP <= 4 ? 5 : 1)))
 void attn_rope_scores_kernel(AttnRopeArgs r) {
     constexpr int LP = D / 8, PPW = 64 / LP, PER_WAVE = ATT_B / 4, ITERS = PER_WAVE / PPW;
+    constexpr int LH = D / 16, QWAVES = (REP + 64 / LH - 1) / (64 / LH);
     const AttnArgs &a = r.at;
     __shared__ float sc[REP][ATT_B];
     __shared__ u32x4 qk_s[(REP + 1) * (D / 8)];  // the roped query heads, then the key
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int G = lane / LP, L = lane % LP;
+    const int w = wave_id();
+    const int kv_dim = a.n_kv_heads * D;
     const int pos = *a.d_pos;
+    ScoresRopeIn<D, TABLE> in;
+    bool roper = rope_request<D, REP>(r, (int)blockIdx.x % a.n_kv_heads, in);
+    __builtin_amdgcn_sched_barrier(0);  // ahead of the key rows
     const int n = pos + 1;
     const int nb = (n + ATT_B - 1) / ATT_B;
-    const int kv_dim = a.n_kv_heads * D;
     for (int item = blockIdx.x; item < nb * a.n_kv_heads; item += gridDim.x) {
         const int b = item / a.n_kv_heads, g = item - b * a.n_kv_heads;
-        const bool last = b == nb - 1;
-        RopeIn<D> in;
-        const bool roper = rope_request<D, REP>(r, g, pos, last, in);
-        LaneFreq<D> freq{};
-        if constexpr (TABLE) {
-            constexpr int HALF = D / 2;
-            const __amdgpu_buffer_rsrc_t tr = __builtin_amdgcn_make_buffer_rsrc(
-                (void *)r.table, (short)0, 2 * HALF * 4, BUFFER_FLAGS);
-#pragma unroll
-            for (int m = 0; m < RopeShape<D>::NJ; m++) {
-                const int j = lane + 64 * m;  // entries past HALF read as zeros
-                in.cs[m] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                    tr, 4 * (j < HALF ? j : 2 * HALF), 0, 0));
-                in.sn[m] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
-                    tr, 4 * (j < HALF ? HALF + j : 2 * HALF), 0, 0));
-            }
-            __builtin_amdgcn_sched_barrier(0);  // ahead of the key rows
-        } else {
-            freq = lane_freq<D>(r.inv_freq);
+        if (item != (int)blockIdx.x) {
+            __syncthreads();  // the previous item's LDS has been read
+            roper = rope_request<D, REP>(r, g, in);
         }
+        const int lane = tid_x() & 63, G = lane / LP, L = lane % LP;  // not held over the loop
         u32x4 kv[ITERS];
-#pragma unroll
-        for (int it = 0; it < ITERS; it++) {
-            const int t = b * ATT_B + w * PER_WAVE + it * PPW + G;
-            kv[it] = t < pos ? ld16_nt(a.kc + (size_t)t * kv_dim + g * D + 8 * L) : u32x4{0, 0, 0, 0};
-        }
-        // the table while the rows stream (arithmetic only)
-        if (!TABLE && roper) rope_table<D>(pos, freq, in.cs, in.sn);
-        __syncthreads();  // qk_s of the previous item has been read
-        if (roper) rope_finish<D, REP>(r, g, pos, in, qk_s, qk_s + REP * (D / 8));
+        request_rows<D, ITERS>(a.kc, kv_dim, b, g, pos, w * PER_WAVE + G, L, kv);
+        asm volatile("" ::: "memory");  // the key rows are requested before the rotation
+        if (roper && (w < QWAVES || b == nb - 1))
+            rope_finish<D, REP, TABLE>(r, g, pos, in, qk_s, qk_s + REP * (D / 8));
         __syncthreads();
 #pragma unroll
         for (int it = 0; it < ITERS; it++)
