@@ -2571,6 +2571,7 @@ struct SampleSlot {
     unsigned done;   // workgroups of the second launch that have published their sums
     float pad[30];
     float sums[SAMPLE_T];
+    float maxes[SAMPLE_WGS];  // of a step's slot: parts of the row's max
 };
 static __device__ SampleSlot g_sample_slots[SAMPLE_SLOTS];
 
@@ -2735,14 +2736,34 @@ __global__ __launch_bounds__(SAMPLE_T) void sample_kernel(int *out, const bf16 *
     if (t == 0) *out = chosen;
 }
 
-// A call that knows where the row's max is (a decode step that has its argmax) and has a slot of its
-// own needs no first launch: *out holds the index of the max, and the drawn token is also handed to the
-// host, with the step's error flag, in the two pinned words at mail.
+// A decode step draws with a slot of its own. If it has its argmax, *out holds the index of the max and
+// no other launch is needed; else sample_max_kernel has left the max in parts. The drawn token is also
+// handed to the host, with the step's error flag, in the two pinned words at mail.
 struct SampleStep {
     SampleSlot *slot;  // NULL: the slot and the max are in the ticket
+    int parts;         // the max is in the slot's parts
     int *mail;
     const int *err;
 };
+
+// Workgroup w's part of the row's max. vec: x is 16-byte aligned.
+__global__ __launch_bounds__(256) void sample_max_kernel(SampleSlot *slot, const bf16 *x, int n, int vec) {
+    __shared__ float wmax[4];
+    const int t0 = blockIdx.x * 256 + threadIdx.x, stride = SAMPLE_WGS * 256;
+    float m = -__builtin_huge_valf();
+    const int n_chunks = vec ? n / 8 : 0;
+    for (int c = t0; c < n_chunks; c += stride) {
+        const u32x4 v = ld16(x + 8 * (size_t)c);
+#pragma unroll
+        for (int e = 0; e < 8; e++) m = fmaxf(m, elem(v, e));
+    }
+    for (int i = 8 * n_chunks + t0; i < n; i += stride) m = fmaxf(m, bf2f(x[i]));
+    m = wave_max(m);
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        slot->maxes[blockIdx.x] = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+}
 
 // Workgroup w: the sums of chunks [w SAMPLE_ROWS, (w + 1) SAMPLE_ROWS). All threads compute the
 // weights of a piece of each chunk into LDS (four chunks per wave, one lane per weight), then lane r
@@ -2774,7 +2795,10 @@ __global__ __launch_bounds__(256) void sample_sums_kernel(int *out, const bf16 *
     const uint32_t ticket = (uint32_t)*out;
     SampleSlot *slot = step.slot;
     float mx;
-    if (slot) {  // an index past the row (no element is a number): the max of no numbers
+    static_assert(SAMPLE_WGS == 64, "a lane per part");
+    if (slot && step.parts) {
+        mx = wave_max(slot->maxes[lane]);
+    } else if (slot) {  // an index past the row (no element is a number): the max of no numbers
         mx = ticket < (uint32_t)n ? bf2f(x[ticket]) : -__builtin_huge_valf();
     } else {
         // not a ticket: the first launch has drawn
@@ -2871,11 +2895,16 @@ extern "C" void sample_forward(int *out, const bf16 *x, int n, float inv_temp, f
 }
 
 size_t sample_slot_bytes() { return sizeof(SampleSlot); }
+bool sample_takes_one_launch(int n) { return n <= SAMPLE_ALONE; }
 
-bool sample_known_max(int *out, const bf16 *x, int n, float inv_temp, float u, void *slot, int *mail,
-                      const int *err, hipStream_t stream) {
+bool sample_step(int *out, const bf16 *x, int n, float inv_temp, float u, bool argmax_in_out,
+                 void *slot, int *mail, const int *err, hipStream_t stream) {
+    if (!argmax_in_out) {
+        sample_max_kernel<<<SAMPLE_WGS, 256, 0, stream>>>((SampleSlot *)slot, x, n, aligned16(x) ? 1 : 0);
+        if (!LAUNCH_OK()) return false;
+    }
     sample_sums_kernel<<<SAMPLE_WGS, 256, 0, stream>>>(
-        out, x, n, inv_temp, u, SampleStep{(SampleSlot *)slot, mail, err});
+        out, x, n, inv_temp, u, SampleStep{(SampleSlot *)slot, argmax_in_out ? 0 : 1, mail, err});
     return LAUNCH_OK();
 }
 

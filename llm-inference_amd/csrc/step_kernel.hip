@@ -1773,15 +1773,15 @@ struct Shape {
     // split, tokens/s): 0.6B 384 1778 / 1713, 448 1693 / 1707, 512 1480 / 1683; 1.7B 320 1016 /
     // 993, 384 987 / 990, 448 958 / 985; 4B 448 517 / 504, 512 488 / 511.
     static constexpr int SPLIT_BLOCKS = H <= 1024 ? 8 : H <= 2048 ? 7 : 9;
-    // STEP_AUTO's switch to the hipGraph step (at most the kernel's longest history), from the
-    // split instance's and the graph's per-token times on MI355X (64 greedy tokens after an
-    // N(0, 1) cache; split / graph tokens/s): 0.6B 4096 1450 / 1138, 8128 1213 / 1032; 1.7B
-    // 4096 865 / 826, 5120 792 / 809, 6144 791 / 792, 7168 790 / 779, 8128 802 / 766; 4B 4096
-    // 467-477 / 464-467, 5120 442 / 460, 6144 448 / 449, 7168 438 / 444, 8192 432-438 / 433-434.
-    // The graph leads by at most 4%, between ~5000 and ~7500 positions at 1.7B and 4B, so the
-    // kernel runs every position it holds (one launch per generate call). The small test shape
-    // keeps a switch (736) so that a generate_greedy crossing it is exercised.
-    static constexpr int SWITCH_POS = H < 1024 ? 736 : 1 << 30;
+    // STEP_AUTO's switch to the hipGraph step (at most the kernel's longest history): the crossover of
+    // the split instance's and the graph's time per token, measured on MI355X (us, 32 greedy tokens after
+    // an N(0, 1) cache; split / graph): 4B 4000 2038 / 2056, 4100 2076 / 2070, 4300 2132 / 2069, 5000
+    // 2237 / 2080, 8200 2250 / 2200, 10000 2385 / 2230; 1.7B 4250 1131 / 1160, 4416 1158 / 1166, 4500
+    // 1172 / 1160, 5000 1270 / 1153, 8300 1260 / 1246, 10000 1319 / 1263; 0.6B: the kernel at every length
+    // it holds (8200 774 / 947). From 64 blocks on a half-slot of the kernel runs a second item, while the
+    // graph's passes grow smoothly. The small test shape keeps a switch (736) so that a generate_greedy
+    // crossing it is exercised.
+    static constexpr int SWITCH_POS = H < 1024 ? 736 : H <= 1024 ? 1 << 30 : H <= 2048 ? 4480 : 4096;
     // The split attention's statistics (block and global max and sum) reduce with their xor-4
     // and xor-8 steps through ds_swizzle (LDS8) where two query heads share a kv head, through
     // DPP at 4B (four): 0.6B after 8192 positions 1235-1237 tokens/s against 1185-1194 with DPP;
