@@ -1407,7 +1407,10 @@ __device__ __forceinline__ void pv_item(const AttnArgs &a, int b, int g, int n, 
     // for them and runs while the values stream. Unconditional (clamped indices), so no branch joins
     // before the value requests.
     constexpr int MAXC = 4;  // chunks of 64 block statistics held in registers
-    const int wu = wave_id();
+    // (which waves have heads turns with the workgroups of a CU, 256 apart, for heads of 128 and more:
+    // those with REP < 4 leave waves idle here; 8 heads on 1 of 128 at 2000 positions 21.3 -> 21.1 us a
+    // block, the 1.7B hipGraph step after 5000 1152 -> 1146 us; of 64 it measured 0.8% slower)
+    const int wu = (wave_id() + (D >= 128 ? (int)(blockIdx.x >> 8) : 0)) & 3;
     float mv0[MAXC], sv0[MAXC], s_t0;
     {
         const int h = g * REP + (wu < REP ? wu : 0);
@@ -2151,7 +2154,7 @@ extern "C" void qk_norm_rope_attention_one_pass(bf16 *out, const bf16 *q, const 
 // partials with agent scope, and the items of the T last blocks of each kv head then combine: item
 // nb - T + j adds, in block order, the partials of columns [j C, (j + 1) C) of the kv head's REP * D
 // (C = REP * D / T), polling the words until none is marked. T is the largest power of two <=
-// min(nb, REP * D / PVC_COLS, PVC_MAX_WAIT / n_kv_heads). The mark travels in the word itself and is
+// min(nb, REP * D / PVC_COLS, PVC_MAX_T, PVC_MAX_WAIT / n_kv_heads). The mark travels in the word itself and is
 // set by the launch before, so nothing is counted or kept from call to call, and the words stay 32
 // bits wide. One workgroup per item of the longest history; only the T * n_kv_heads combine items
 // wait, fewer than the workgroups the device holds at once, and every other item runs to its end,
@@ -2170,6 +2173,8 @@ extern "C" void qk_norm_rope_attention_one_pass(bf16 *out, const bf16 *q, const 
 // fewest columns of a combine item (4B after 8192 positions: 431.2-431.8 tokens/s; 8 columns
 // 428.5-428.8, 32 columns 418.5-418.6)
 constexpr int PVC_COLS = 16;
+// combine items per kv head (32 heads on 4 of 256 at 12000 positions: 64 39.6 us a block, 128 41.5, 32 41.3)
+constexpr int PVC_MAX_T = 64;
 constexpr int PVC_MAX_WAIT = 512;   // combine items of a launch (the device holds >= 1024 workgroups)
 constexpr int PVC_MAXGRID = 8192;   // items (blocks x kv heads) of the longest history
 
@@ -2199,7 +2204,9 @@ __global__ __launch_bounds__(256) void attn_pv_combine_kernel(AttnArgs a) {
                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     });
     int T = 1;
-    while (2 * T <= nb && 2 * T * PVC_COLS <= COLS && 2 * T * a.n_kv_heads <= PVC_MAX_WAIT) T *= 2;
+    while (2 * T <= nb && 2 * T <= PVC_MAX_T && 2 * T * PVC_COLS <= COLS &&
+           2 * T * a.n_kv_heads <= PVC_MAX_WAIT)
+        T *= 2;
     if (b < nb - T) return;
     const int nc = COLS / T, c0 = (b - (nb - T)) * nc, nq = nc / 4;  // powers of two
     // blocks per staged chunk: a column's partials lie side by side (read 16 bytes at a time), the
