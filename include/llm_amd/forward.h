@@ -134,7 +134,8 @@ typedef struct {
                                head below this many blocks of 64 positions of history, and split
                                over (kv head, block) items from it on (1..128; set by
                                capture_graph to the shapes' measured crossover) */
-    void *sample_slot;      /* the temperature draw's chunk sums (zeroed at allocation) */
+    void *sample_slot;      /* the temperature draw's parts of the max and chunk sums
+                               (zeroed at allocation) */
     int *mail;              /* pinned host words: the last sampled token, the error flag */
     int *mail_dev;          /* their device address */
 } RunState;

