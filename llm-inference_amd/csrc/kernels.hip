@@ -2164,7 +2164,8 @@ extern "C" void qk_norm_rope_attention_one_pass(bf16 *out, const bf16 *q, const 
 // Bound by its chain (statistics, exponentials, the products, the hand-over, the in-order sums)
 // rather than by the value stream: 32 heads on 8 kv heads of 128 at 8300 positions (17 MB of values)
 // 10.6 us, against 8.1 + 5.4 us as two launches; 16 on 8 at 260 positions 5.0 against 3.9 + 3.0; 8 on
-// 4 of 64 at 12345 positions 8.6 against 5.1 + 6.9. In the hipGraph step it replaces a form whose
+// 4 of 64 at 12345 positions 8.6 against 5.1 + 6.9. With the statistics by chunk count and the additions
+// read ahead: 9.6, 4.7 and 6.8 us. In the hipGraph step it replaces a form whose
 // partials were tagged 64-bit words with a launch counter per workgroup, at head_dim 128 only:
 // Qwen3-0.6B after 300 positions 754 -> 730 us per token, 4B after 8192 2276 -> 2268, 8 on 4 heads
 // of 64 after 300 positions (12 layers of 512) 258 -> 243.
@@ -2749,7 +2750,7 @@ __global__ __launch_bounds__(SAMPLE_T) void sample_kernel(int *out, const bf16 *
 }
 
 // A decode step draws with a slot of its own, in which sample_max_kernel has left the row's max in
-// parts (2 us, against 6 with one workgroup). The drawn token is also handed to the host, with the
+// parts (traced in a sampled 4B decode: 4.5 us, against 5.6 with one workgroup). The drawn token is also handed to the host, with the
 // step's error flag, in the two pinned words at mail.
 struct SampleStep {
     SampleSlot *slot;  // NULL: the slot and the max are in the ticket
