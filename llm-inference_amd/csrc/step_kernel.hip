@@ -1952,8 +1952,8 @@ int step_kernel_split_blocks(const Config *cfg) {
     return 0;
 }
 
-// Measured on MI355X, 5-token prompt then 128-256 tokens: 0.6B 2356 tokens/s (step kernel)
-// against 1278 (hipGraph), 1.7B 1121 against 893, 4B 578 against 492.
+// Measured on MI355X, 32 tokens from position 5: 0.6B 373 us per token (step kernel) against 724
+// (hipGraph), 1.7B 874 against 1051, 4B 1603 against 1925.
 int step_kernel_switch_pos(const Config *cfg) {
     int sw = 0;
 #define SWITCH(S)                                                                           \
