@@ -32,7 +32,7 @@ bool attention_one_pass_launch(bf16 *out, const bf16 *q, const bf16 *k, const bf
                                int max_seq, float scale, hipStream_t stream);
 
 // attention_forward, reporting whether it launched; err: the step's device error flag (set to 1 for
-// a position outside the cache and to 2 if a wait between workgroups times out), or NULL.
+// a position outside the cache), or NULL.
 bool attention_launch(bf16 *out, const bf16 *q, const bf16 *key_cache, const bf16 *value_cache,
                       float *att, int n_heads, int n_kv_heads, int head_dim, const int *d_pos,
                       int max_seq, float scale, hipStream_t stream, int *err = nullptr);

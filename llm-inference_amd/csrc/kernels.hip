@@ -1001,6 +1001,7 @@ __device__ __forceinline__ void ld_lds16(const float *p, float (&v)[16]) {
 }
 
 constexpr int ATT_B = 64;  // positions per block
+constexpr int ATTN_MAXGRID = 8192;  // workgroups of a pass
 
 struct AttnArgs {
     bf16 *out;
@@ -1013,22 +1014,14 @@ struct AttnArgs {
     const int *d_pos;
     int n_heads, n_kv_heads, max_seq, max_blocks;
     float scale;
-    int mark;    // the scores pass marks the item's partials as not yet written (ATT_UNWRITTEN)
-    int *err;    // the step's error flag (set to 2 when a wait times out), or NULL
+    int *err;    // the step's error flag (set to 1 for a position outside the cache), or NULL
 };
 
-// A block partial that attn_pv_combine_kernel has not stored yet: a NaN that no sum of products of
-// bf16 values produces (a NaN made from bf16 inputs has a payload with a zero low half); should one
-// appear all the same, it is stored as the NaN next to it.
-constexpr uint32_t ATT_UNWRITTEN = 0xffffffffu;
-
-// Marks the partials of block b of the kv head's REP query heads.
-template <int D, int REP>
-__device__ __forceinline__ void mark_partials(const AttnArgs &a, int b, int g) {
-    constexpr int Q = D / 4;  // 16-byte stores per head
-    for (int i = tid_x(); i < REP * Q; i += 256)
-        st16(a.partial + ((size_t)(g * REP + i / Q) * a.max_blocks + b) * D + 4 * (i % Q),
-             u32x4{ATT_UNWRITTEN, ATT_UNWRITTEN, ATT_UNWRITTEN, ATT_UNWRITTEN});
+// A block's max in the statistics. It is one of the scores, which are bf16 values: the low half of its
+// word is zero after the scores pass, and for block 0 of a kv head's first query head it then counts
+// the head's items that have stored their partials (attn_pv_combine_kernel).
+__device__ __forceinline__ float block_max(const float *st, int b) {
+    return __uint_as_float(__float_as_uint(st[2 * b]) & 0xffff0000u);
 }
 
 static size_t ceil_div(size_t a, size_t b) { return (a + b - 1) / b; }
@@ -1107,7 +1100,6 @@ __global__ __launch_bounds__(256) void attn_scores_kernel(AttnArgs a) {
             }
         }
         __syncthreads();
-        if (a.mark) mark_partials<D, REP>(a, b, g);
         for (int r = w; r < REP; r += 4) {
             const bool v = b * ATT_B + lane < n;
             const float s = v ? sc[r][lane] : -__builtin_huge_valf();
@@ -1371,7 +1363,6 @@ void attn_rope_scores_kernel(AttnRopeArgs r) {
             }
         }
         __syncthreads();
-        if (a.mark) mark_partials<D, REP>(a, b, g);
         for (int q = w; q < REP; q += 4) {
             const bool v = b * ATT_B + lane < n;
             const float s = v ? sc[q][lane] : -__builtin_huge_valf();
@@ -1419,7 +1410,7 @@ __device__ __forceinline__ void pv_item(const AttnArgs &a, int b, int g, int n, 
 #pragma unroll
         for (int c = 0; c < MAXC; c++) {
             const int bi = min(c * 64 + lane, nb - 1);
-            mv0[c] = st[2 * bi];
+            mv0[c] = block_max(st, bi);
             sv0[c] = st[2 * bi + 1];
         }
     }
@@ -1477,7 +1468,7 @@ __device__ __forceinline__ void pv_item(const AttnArgs &a, int b, int g, int n, 
 #pragma unroll
             for (int c = 0; c < MAXC; c++) {
                 const int bi = min(c * 64 + lane, nb - 1);
-                mv[c] = st[2 * bi];
+                mv[c] = block_max(st, bi);
                 sv[c] = st[2 * bi + 1];
             }
             p_s[r][lane] = prob_of(s_t, mv, sv);
@@ -1491,11 +1482,11 @@ __device__ __forceinline__ void pv_item(const AttnArgs &a, int b, int g, int n, 
         float M = -__builtin_huge_valf(), sum = 0.0f;
         for (int c0 = 0; c0 < nb; c0 += 64) {
             const int bi = c0 + lane;
-            M = fmaxf(M, wave_max(bi < nb ? st[2 * bi] : -__builtin_huge_valf()));
+            M = fmaxf(M, wave_max(bi < nb ? block_max(st, bi) : -__builtin_huge_valf()));
         }
         for (int c0 = 0; c0 < nb; c0 += 64) {
             const int bi = c0 + lane;
-            const float term = bi < nb ? st[2 * bi + 1] * exp_f32(st[2 * bi] - M) : 0.0f;
+            const float term = bi < nb ? st[2 * bi + 1] * exp_f32(block_max(st, bi) - M) : 0.0f;
             const float cs = wave_sum(term);
             sum = c0 == 0 ? cs : sum + cs;
         }
@@ -1543,7 +1534,6 @@ __device__ __forceinline__ void pv_item(const AttnArgs &a, int b, int g, int n, 
         const float v = ((red[0][r][d] + red[1][r][d]) + red[2][r][d]) + red[3][r][d];
         store(((size_t)(g * REP + r) * a.max_blocks + b) * D + d, v);
     }
-    __syncthreads();
 }
 
 template <int D, int REP>
@@ -1556,6 +1546,7 @@ __global__ __launch_bounds__(256) void attn_pv_kernel(AttnArgs a) {
         const int b = item / a.n_kv_heads, g = item - b * a.n_kv_heads;
         pv_item<D, REP>(a, b, g, n, nb, p_s, red,
                         [&](size_t i, float v) { a.partial[i] = v; });
+        __syncthreads();
     }
 }
 
@@ -2150,44 +2141,39 @@ extern "C" void qk_norm_rope_attention_one_pass(bf16 *out, const bf16 *q, const 
 
 // ------------------------------------------------------------------------------------------
 // Passes 2 and 3 in one launch (attn_pv_kernel followed by attn_combine_kernel, the same bits).
-// The scores pass has marked every block's partials ATT_UNWRITTEN; every item stores its block
-// partials with agent scope, and the items of the T last blocks of each kv head then combine: item
-// nb - T + j adds, in block order, the partials of columns [j C, (j + 1) C) of the kv head's REP * D
-// (C = REP * D / T), polling the words until none is marked. T is the largest power of two <=
-// min(nb, REP * D / PVC_COLS, PVC_MAX_T, PVC_MAX_WAIT / n_kv_heads). The mark travels in the word itself and is
-// set by the launch before, so nothing is counted or kept from call to call, and the words stay 32
-// bits wide. One workgroup per item of the longest history; only the T * n_kv_heads combine items
-// wait, fewer than the workgroups the device holds at once, and every other item runs to its end,
-// so the waits end. They are bounded all the same: on a timeout the kernel finishes with what it
-// read (NaN), and sets *err where there is one.
+// Every item stores its block partials with agent scope and then counts itself in the low half of the
+// max of its kv head's first block (block_max; the scores pass has left a zero there). The item that
+// completes the count adds the kv head's partials in block order. No workgroup waits for another one:
+// the launch ends whatever else runs on the device and however few of its workgroups fit at once, and
+// nothing is kept from call to call.
 //
-// Bound by its chain (statistics, exponentials, the products, the hand-over, the in-order sums)
-// rather than by the value stream: 32 heads on 8 kv heads of 128 at 8300 positions (17 MB of values)
-// 10.6 us, against 8.1 + 5.4 us as two launches; 16 on 8 at 260 positions 5.0 against 3.9 + 3.0; 8 on
-// 4 of 64 at 12345 positions 8.6 against 5.1 + 6.9. With the statistics by chunk count and the additions
-// read ahead: 9.6, 4.7 and 6.8 us. In the hipGraph step it replaces a form whose
-// partials were tagged 64-bit words with a launch counter per workgroup, at head_dim 128 only:
-// Qwen3-0.6B after 300 positions 754 -> 730 us per token, 4B after 8192 2276 -> 2268, 8 on 4 heads
-// of 64 after 300 positions (12 layers of 512) 258 -> 243.
+// Bound by its chain (statistics, exponentials, the products, the count, the in-order sums) rather
+// than by the value stream, and at long histories by the one CU that reads a kv head's partials, at
+// some 50 GB/s. The line of PVC_MAX_FLOATS, from attention_forward of a full history in us, one launch
+// / two (heads on kv heads of head_dim, blocks):
+//   16 on 8 of 128: 8 blocks 7.6 / 8.5, 64 10.7 / 12.2, 128 14.6 / 15.7, 192 19.2 / 19.7, 256 30.5 / 23.2
+//   32 on 8 of 128: 8 7.6 / 9.2, 64 12.5 / 12.8, 128 17.1 / 17.3, 192 22.5 / 22.5, 256 33.9 / 26.4
+//   4 on 1 of 128: 8 8.0 / 8.6, 64 10.5 / 10.4, 96 12.3 / 11.3; 8 on 1: 16 10.3 / 11.0, 64 13.0 / 12.1
+//   64 on 8 of 256: 8 12.9 / 13.5, 16 14.2 / 14.2, 32 16.7 / 15.8; 1 on 1 of 64: 96 8.8 / 9.0, 128 10.2 / 9.7
+// The host knows the longest history only; shorter ones in the same caches gain most from one launch
+// (16 on 8 of 128 at 260 positions of 4096: 6.4 / 7.5), so the lines lie past the last full history
+// that gains. Past PVC_MAX_ITEMS the workgroups, which stay until their stores are acknowledged, no
+// longer fit the device at once (the 256-block figures of 8 kv heads).
 // ------------------------------------------------------------------------------------------
 
-// fewest columns of a combine item (4B after 8192 positions: 431.2-431.8 tokens/s; 8 columns
-// 428.5-428.8, 32 columns 418.5-418.6)
-constexpr int PVC_COLS = 16;
-// combine items per kv head (32 heads on 4 of 256 at 12000 positions: 64 39.6 us a block, 128 41.5, 32 41.3)
-constexpr int PVC_MAX_T = 64;
-constexpr int PVC_MAX_WAIT = 512;   // combine items of a launch (the device holds >= 1024 workgroups)
-constexpr int PVC_MAXGRID = 8192;   // items (blocks x kv heads) of the longest history
+constexpr int PVC_MAX_FLOATS = 49152;  // partials of a kv head: blocks of the longest history x REP * D
+constexpr int PVC_MAX_BLOCKS = 128;
+constexpr int PVC_MAX_ITEMS = 1280;    // blocks x kv heads
+static_assert(PVC_MAX_BLOCKS < 0x10000, "the count of a kv head's items fits 16 bits");
 
 template <int D, int REP>
 __global__ __launch_bounds__(256) void attn_pv_combine_kernel(AttnArgs a) {
     constexpr int COLS = REP * D;
-    constexpr int STAGE = 4 * REP * D > 4096 ? 4 * REP * D : 4096;  // floats
-    constexpr int CPT = (COLS + 255) / 256;  // columns of a thread when one item combines all
-    constexpr int K = 4;                     // 16-byte words of a thread in flight while polling
+    constexpr int C = COLS > 256 ? COLS / 256 : 1;  // columns of a thread in the combine
+    constexpr int U = 32 / C;                       // blocks it requests at a time
     __shared__ float p_s[REP][ATT_B];
-    __shared__ __align__(16) float stage[STAGE];  // the PV quarter sums, then the staged partials
-    float(&red)[4][REP][D] = *reinterpret_cast<float(*)[4][REP][D]>(stage);
+    __shared__ float red[4][REP][D];
+    __shared__ int s_last;
     const int n = *a.d_pos + 1;
     const int nb = (n + ATT_B - 1) / ATT_B;
     if (n <= 0 || n > a.max_seq) {  // no history, or none the caches can hold: zeros
@@ -2200,101 +2186,74 @@ __global__ __launch_bounds__(256) void attn_pv_combine_kernel(AttnArgs a) {
     if ((int)blockIdx.x >= nb * a.n_kv_heads) return;  // the grid holds every item: one each
     const int b = blockIdx.x / a.n_kv_heads, g = blockIdx.x - b * a.n_kv_heads;
     pv_item<D, REP>(a, b, g, n, nb, p_s, red, [&](size_t i, float v) {
-        const uint32_t u = __float_as_uint(v);
-        __hip_atomic_store(gptr((uint32_t *)a.partial + i), u == ATT_UNWRITTEN ? u - 1 : u,
-                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(gptr(a.partial + i), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     });
-    int T = 1;
-    while (2 * T <= nb && 2 * T <= PVC_MAX_T && 2 * T * PVC_COLS <= COLS &&
-           2 * T * a.n_kv_heads <= PVC_MAX_WAIT)
-        T *= 2;
-    if (b < nb - T) return;
-    const int nc = COLS / T, c0 = (b - (nb - T)) * nc, nq = nc / 4;  // powers of two
-    // blocks per staged chunk: a column's partials lie side by side (read 16 bytes at a time), the
-    // columns an odd multiple of 16 bytes apart where there is room
-    const int cb = STAGE / nc >= 32 ? STAGE / nc - 4 : STAGE / nc;
-    const int qsh = __builtin_ctz(nq);
+    // The partials are written through to the level all XCDs share: once every wave's stores are
+    // acknowledged there, the count needs no release of its own (which writes back the whole L2).
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t *count = (uint32_t *)(a.stats + (size_t)g * REP * a.max_blocks * 2);
+        s_last = (int)(__hip_atomic_fetch_add(gptr(count), 1u, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT) & 0xffff) == nb - 1;
+    }
+    __syncthreads();
+    if (!s_last) return;
+    // the partials are read with agent scope too, past this XCD's own copies of those lines
+    const int c0 = threadIdx.x * C;  // columns c0 .. c0 + C - 1 of the kv head's REP * D
+    if (c0 >= COLS) return;
     // the kv head's partials as one buffer: REP heads of max_blocks rows of D
     const __amdgpu_buffer_rsrc_t pr = __builtin_amdgcn_make_buffer_rsrc(
         (void *)(a.partial + (size_t)g * REP * a.max_blocks * D), (short)0,
         REP * a.max_blocks * D * 4, BUFFER_FLAGS);
-    float acc[CPT];
+    const int at = (c0 / D * a.max_blocks * D + c0 % D) * 4;
+    float acc[C], v[2][U][C];
 #pragma unroll
-    for (int k = 0; k < CPT; k++) acc[k] = -0.0f;  // -0 + x is x, also for x = -0
-    for (int b0 = 0; b0 < nb; b0 += cb) {
-        const int cnt = min(cb, nb - b0), total = cnt << qsh;
-        for (int base = 0; base < total; base += 256 * K) {
-            u32x4 v[K];
-            int off[K];
+    for (int c = 0; c < C; c++) acc[c] = -0.0f;  // -0 + x is x, also for x = -0
+    const auto request = [&](int b0, float (&to)[U][C]) {  // past the end: the last block again
 #pragma unroll
-            for (int k = 0; k < K; k++) {
-                // word quad i: block b0 + i / nq, columns c0 + 4 (i % nq) .. + 3 (past the end: the
-                // last quad again)
-                const int i = min(base + (int)threadIdx.x + 256 * k, total - 1);
-                const int c = c0 + 4 * (i & (nq - 1)), q = c / D;
-                off[k] = ((q * a.max_blocks + b0 + (i >> qsh)) * D + c - q * D) * 4;
-            }
-            long long spins = 0;
-            for (;;) {
-                bool fresh = true;
+        for (int u = 0; u < U; u++) {
+            const int row = min(b0 + u, nb - 1) * D * 4;
+            if constexpr (C == 1) {
+                to[u][0] =
+                    __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(pr, at, row, BUFFER_SC1));
+            } else if constexpr (C == 2) {
+                const auto w = __builtin_amdgcn_raw_buffer_load_b64(pr, at, row, BUFFER_SC1);
+                to[u][0] = __uint_as_float(w[0]);
+                to[u][1] = __uint_as_float(w[1]);
+            } else {
 #pragma unroll
-                for (int k = 0; k < K; k++)
-                    v[k] = __builtin_amdgcn_raw_buffer_load_b128(pr, off[k], 0, BUFFER_SC1);
-#pragma unroll
-                for (int k = 0; k < K; k++)
-                    fresh &= v[k].x != ATT_UNWRITTEN && v[k].y != ATT_UNWRITTEN &&
-                             v[k].z != ATT_UNWRITTEN && v[k].w != ATT_UNWRITTEN;
-                if (fresh) break;
-                if ((++spins & 15) == 0 &&
-                    (a.err ? wait_gives_up(spins, OP_SPIN_LIMIT, a.err) : spins > OP_SPIN_LIMIT))
-                    break;
-                asm volatile("" ::: "memory");  // read the words again
-            }
-#pragma unroll
-            for (int k = 0; k < K; k++) {
-                const int i = base + (int)threadIdx.x + 256 * k;
-                if (i < total) {
-                    float *at = stage + 4 * (i & (nq - 1)) * cb + (i >> qsh);
-#pragma unroll
-                    for (int e = 0; e < 4; e++)
-                        at[e * cb] = __uint_as_float(e == 0 ? v[k].x : e == 1 ? v[k].y : e == 2 ? v[k].z : v[k].w);
+                for (int c = 0; c < C; c += 4) {
+                    const u32x4 w =
+                        __builtin_amdgcn_raw_buffer_load_b128(pr, at + 4 * c, row, BUFFER_SC1);
+                    to[u][c] = __uint_as_float(w.x);
+                    to[u][c + 1] = __uint_as_float(w.y);
+                    to[u][c + 2] = __uint_as_float(w.z);
+                    to[u][c + 3] = __uint_as_float(w.w);
                 }
             }
         }
-        __syncthreads();
+    };
+    const auto add = [&](int b0, const float (&from)[U][C]) {
 #pragma unroll
-        for (int k = 0; k < CPT; k++) {
-            const int c = threadIdx.x + 256 * k;
-            if (c < nc) {
-                // in block order; 16 are added while the next 16 are read
-                const float *col = stage + c * cb;
-                const int whole = cnt & ~15;
-                float v[16], next[16];
-                if (whole) ld_lds16(col, v);
-                for (int j = 0; j < whole; j += 16) {
-                    ld_lds16(col + min(j + 16, cb - 16), next);
+        for (int u = 0; u < U; u++) {
+            if (b0 + u >= nb) break;
 #pragma unroll
-                    for (int u = 0; u < 16; u++) acc[k] += v[u];
-#pragma unroll
-                    for (int u = 0; u < 16; u++) v[u] = next[u];
-                }
-#pragma unroll
-                for (int u = 0; u < 15; u++) v[u] = col[min(whole + u, cnt - 1)];
-#pragma unroll
-                for (int u = 0; u < 15; u++)
-                    if (whole + u < cnt) acc[k] += v[u];
-            }
+            for (int c = 0; c < C; c++) acc[c] += from[u][c];
         }
-        __syncthreads();
+    };
+    request(0, v[0]);
+    for (int b0 = 0; b0 < nb; b0 += 2 * U) {
+        if (b0 + U < nb) request(b0 + U, v[1]);
+        add(b0, v[0]);
+        if (b0 + 2 * U < nb) request(b0 + 2 * U, v[0]);
+        add(b0 + U, v[1]);
     }
 #pragma unroll
-    for (int k = 0; k < CPT; k++)
-        if ((int)threadIdx.x + 256 * k < nc)
-            a.out[(size_t)g * COLS + c0 + threadIdx.x + 256 * k] = (bf16)f2bf(acc[k]);
+    for (int c = 0; c < C; c++) a.out[(size_t)g * COLS + c0 + c] = (bf16)f2bf(acc[c]);
 }
 
-// The scores pass, then PV and combine: one launch where the grid holds every item of the longest
-// history (a.mark, set by attention_args), else the two kernels.
+// The scores pass, then PV and combine in one launch or two.
 template <int D, int REP>
 static void launch_attention_t(const AttnArgs &a, int grid, hipStream_t stream,
                                const AttnRopeArgs *rope = nullptr) {
@@ -2305,7 +2264,8 @@ static void launch_attention_t(const AttnArgs &a, int grid, hipStream_t stream,
     else
         attn_scores_kernel<D, REP><<<grid, 256, 0, stream>>>(a);
     if (!LAUNCH_OK()) return;
-    if (a.mark) {
+    if (a.max_blocks <= PVC_MAX_BLOCKS && a.max_blocks * REP * D <= PVC_MAX_FLOATS &&
+        (long)a.max_blocks * a.n_kv_heads <= PVC_MAX_ITEMS) {
         attn_pv_combine_kernel<D, REP><<<grid, 256, 0, stream>>>(a);
         LAUNCH_OK();
         return;
@@ -2415,8 +2375,7 @@ static bool attention_args(AttnArgs &a, int &grid, bf16 *out, const bf16 *q,
     // the same wave of workgroups (a fixed cap made the last few items of a long history a second
     // wave that doubled the kernel time); items beyond the current history exit at once
     const long items = (long)a.max_blocks * n_kv_heads;
-    grid = (int)(items < PVC_MAXGRID ? items : PVC_MAXGRID);
-    a.mark = items <= PVC_MAXGRID;
+    grid = (int)(items < ATTN_MAXGRID ? items : ATTN_MAXGRID);
     a.err = err;
     return true;
 }

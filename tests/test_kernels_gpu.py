@@ -421,6 +421,78 @@ def test_attention_one_launch_combine(gpu, oracle, hq, hkv, D, pos, max_seq):
     assert np.array_equal(got, want)
 
 
+# histories around the combine's batches of blocks (32 columns' worth: 32, 16, 8 and 4 blocks at 64-256,
+# 512, 1024 and 2048 columns of a kv head), and the longest that one launch takes
+@pytest.mark.parametrize("hq,hkv,D,max_seq,blocks", [
+    (2, 2, 64, 8192, (1, 31, 32, 33, 64, 65, 127, 128)), (16, 8, 128, 8192, (32, 33, 96, 97, 128)),
+    (2, 1, 256, 6144, (15, 16, 17, 32, 33, 96)), (4, 1, 256, 3072, (7, 8, 9, 16, 17, 47, 48)),
+    (16, 2, 256, 1536, (3, 4, 5, 8, 9, 24)), (16, 8, 128, 8193, (128, 129)), (16, 16, 64, 5121, (81,))])
+def test_attention_combine_batches(gpu, oracle, hq, hkv, D, max_seq, blocks):
+    """PV and combine in one launch, and in two just past its limits: bit-identical to the oracle at
+    the first and the last position of each count of blocks, on one workspace that begins as ones."""
+    import torch
+    ident(f"attention combine batches {hq}/{hkv} D{D} of {max_seq}")
+    rng = np.random.default_rng(hq * 10007 + max_seq)
+    kc, vc = rand_bf16(rng, (max_seq, hkv * D)), rand_bf16(rng, (max_seq, hkv * D))
+    kd, vd = dev(kc), dev(vc)
+    floats = gpu.attention_workspace_floats(hq, D, max_seq)
+    att = torch.full((floats,), -1, dtype=torch.int32, device="cuda").view(torch.float32)
+    scale = float(np.float32(1.0 / np.sqrt(D)))
+    for nb in blocks:
+        for pos in {64 * nb - 64, min(64 * nb, max_seq) - 1}:
+            q = rand_bf16(rng, hq * D)
+            out = dev(np.full(hq * D, 0x1234, np.uint16))
+            gpu.attention_forward(out, dev(q), kd, vd, att, hq, hkv, D, dev_i32([pos]), max_seq, scale)
+            want = oracle.attention(q, kc, vc, hq, hkv, D, pos, scale, oracle.GPU_ORDER)
+            assert np.array_equal(host(out), want), pos
+
+
+# the shapes whose last blocks' workgroups are the most and the largest
+@pytest.mark.parametrize("hq,hkv,D,max_seq", [(64, 8, 128, 3072), (64, 8, 256, 1536), (64, 8, 128, 8192),
+                                              (32, 8, 256, 3072)])
+def test_attention_overlapping_streams(gpu, hq, hkv, D, max_seq):
+    """Attention calls of both forms on six streams at once, each with a workspace of its own: every
+    result is that of the same call alone."""
+    import torch
+    ident(f"attention on six streams {hq}/{hkv} D{D} of {max_seq}")
+    g = torch.Generator(device="cuda").manual_seed(hq + D + max_seq)
+    bf = torch.bfloat16
+
+    def normal(*shape):
+        return torch.randn(*shape, generator=g, device="cuda", dtype=bf)
+
+    scale, kvd, n = float(np.float32(1.0 / np.sqrt(D))), hkv * D, 6
+    kc, vc, norm = normal(max_seq, kvd), normal(max_seq, kvd), normal(D)
+    own = [dict(q=normal(hq * D), k=normal(kvd), v=normal(kvd), kc=kc.clone(), vc=vc.clone(),
+                att=torch.empty(gpu.attention_workspace_floats(hq, D, max_seq), device="cuda"),
+                pos=dev_i32([max_seq - 1 - 100 * i]), out=torch.zeros(4, hq * D, device="cuda", dtype=bf))
+           for i in range(n)]
+
+    def call(c, i, row, stream):
+        if i % 2:
+            gpu.qk_norm_rope_attention_forward(c["out"][row], c["q"], c["k"], c["v"], norm, norm,
+                                               c["kc"], c["vc"], c["att"], c["pos"], hq, hkv, D, 1e-6,
+                                               1e6, max_seq, scale, stream=stream)
+        else:
+            gpu.attention_forward(c["out"][row], c["q"], c["kc"], c["vc"], c["att"], hq, hkv, D,
+                                  c["pos"], max_seq, scale, stream=stream)
+
+    torch.cuda.synchronize()
+    for i, c in enumerate(own):
+        call(c, i, 0, None)
+        torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(n)]
+    for row in range(1, 4):
+        for i, c in enumerate(own):
+            call(c, i, row, streams[i])
+    torch.cuda.synchronize()
+    for c in own:
+        rows = c["out"].view(torch.int16)
+        assert c["out"][0].isfinite().all() and c["out"][0].any()
+        for row in range(1, 4):
+            assert torch.equal(rows[0], rows[row])
+
+
 @pytest.mark.parametrize("hq,hkv,D", [(8, 1, 64), (2, 1, 128), (4, 1, 128), (1, 1, 256)])
 def test_attention_statistics_chunks(gpu, oracle, hq, hkv, D):
     """Histories around 1 to 4 chunks of 64 block statistics, and past them, equal the oracle; with
