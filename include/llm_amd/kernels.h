@@ -69,7 +69,8 @@ void qk_norm_rope_forward(bf16 *q, bf16 *k, const bf16 *v, const bf16 *q_norm_w,
  * (head_dim + 2) floats must fit; larger sizes are an error), and calls on one device that use
  * it must not overlap. A smaller `att` is an error. The size is what the runtime reports for the
  * allocation holding `att`, counted from `att` to its end. head_dim in {64, 128, 256};
- * n_heads / n_kv_heads in {1, 2, 4, 8}. */
+ * n_heads / n_kv_heads in {1, 2, 4, 8}. A position outside [0, max_seq) gives zeros; nothing else
+ * is read or written for it. */
 void attention_forward(bf16 *out, const bf16 *q, const bf16 *key_cache, const bf16 *value_cache,
                        float *att, int n_heads, int n_kv_heads, int head_dim, const int *d_pos,
                        int max_seq, float scale, hipStream_t stream);
@@ -122,7 +123,7 @@ void rmsnorm_gate_up_forward(bf16 *act, const bf16 *w_gate, const bf16 *w_up, co
  * instead of four: the per-head QK-norm + RoPE is computed inside the attention's scores pass,
  * per block of positions, while the block's keys stream. q and k are read, not rewritten; k'
  * and v are written to the caches' row *d_pos as qk_norm_rope_forward writes them. `att`, the
- * shapes and alignment are attention_forward's. */
+ * shapes, alignment and positions outside the caches are attention_forward's. */
 void qk_norm_rope_attention_forward(bf16 *out, const bf16 *q, const bf16 *k, const bf16 *v,
                                     const bf16 *q_norm_w, const bf16 *k_norm_w, bf16 *key_cache,
                                     bf16 *value_cache, float *att, const int *d_pos, int n_heads,

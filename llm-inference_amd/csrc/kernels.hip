@@ -1017,6 +1017,16 @@ struct AttnArgs {
     int *err;    // the step's error flag (set to 1 for a position outside the cache), or NULL
 };
 
+// Whether the query's position (n - 1) is one that the caches hold. Where it is not, every pass leaves
+// the caches and the workspace alone, `out` becomes zeros and the step's error flag is set.
+__device__ __forceinline__ bool position_held(const AttnArgs &a, int n) {
+    return n > 0 && n <= a.max_seq;
+}
+__device__ __forceinline__ void position_error(const AttnArgs &a) {
+    if (a.err && blockIdx.x == 0 && threadIdx.x == 0)
+        __hip_atomic_store(gptr(a.err), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // A block's max in the statistics. It is one of the scores, which are bf16 values: the low half of its
 // word is zero after the scores pass, and for block 0 of a kv head's first query head it then counts
 // the head's items that have stored their partials (attn_pv_combine_kernel).
@@ -1066,6 +1076,7 @@ __global__ __launch_bounds__(256) void attn_scores_kernel(AttnArgs a) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int G = lane / LP, L = lane % LP;
     const int n = *a.d_pos + 1;
+    if (!position_held(a, n)) return position_error(a);
     const int nb = (n + ATT_B - 1) / ATT_B;
     const int kv_dim = a.n_kv_heads * D;
     for (int item = blockIdx.x; item < nb * a.n_kv_heads; item += gridDim.x) {
@@ -1323,6 +1334,7 @@ void attn_rope_scores_kernel(AttnRopeArgs r) {
     bool roper = rope_request<D, REP>(r, (int)blockIdx.x % a.n_kv_heads, in);
     __builtin_amdgcn_sched_barrier(0);  // ahead of the key rows
     const int n = pos + 1;
+    if (!position_held(a, n)) return position_error(a);
     const int nb = (n + ATT_B - 1) / ATT_B;
     for (int item = blockIdx.x; item < nb * a.n_kv_heads; item += gridDim.x) {
         const int b = item / a.n_kv_heads, g = item - b * a.n_kv_heads;
@@ -1541,6 +1553,7 @@ __global__ __launch_bounds__(256) void attn_pv_kernel(AttnArgs a) {
     __shared__ float p_s[REP][ATT_B];
     __shared__ float red[4][REP][D];
     const int n = *a.d_pos + 1;
+    if (!position_held(a, n)) return;
     const int nb = (n + ATT_B - 1) / ATT_B;
     for (int item = blockIdx.x; item < nb * a.n_kv_heads; item += gridDim.x) {
         const int b = item / a.n_kv_heads, g = item - b * a.n_kv_heads;
@@ -1585,7 +1598,8 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnArgs a) {
 #pragma unroll
         for (int j = 0; j < PER; j++)
             if ((int)threadIdx.x + 256 * j < n4) ((u32x4 *)part)[threadIdx.x + 256 * j] = v4[j];
-        const int nb = __builtin_amdgcn_readfirstlane((n + ATT_B - 1) / ATT_B);
+        const int nb =
+            __builtin_amdgcn_readfirstlane(position_held(a, n) ? (n + ATT_B - 1) / ATT_B : 0);
         if (b0 >= nb) break;
         const int cnt = min(CB, nb - b0);
         __syncthreads();
@@ -2176,9 +2190,7 @@ __global__ __launch_bounds__(256) void attn_pv_combine_kernel(AttnArgs a) {
     __shared__ int s_last;
     const int n = *a.d_pos + 1;
     const int nb = (n + ATT_B - 1) / ATT_B;
-    if (n <= 0 || n > a.max_seq) {  // no history, or none the caches can hold: zeros
-        if (a.err && threadIdx.x == 0)
-            __hip_atomic_store(gptr(a.err), 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!position_held(a, n)) {
         if ((int)blockIdx.x < a.n_kv_heads)
             for (int i = threadIdx.x; i < COLS; i += 256) a.out[(size_t)blockIdx.x * COLS + i] = 0;
         return;

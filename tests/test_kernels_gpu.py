@@ -447,6 +447,34 @@ def test_attention_combine_batches(gpu, oracle, hq, hkv, D, max_seq, blocks):
             assert np.array_equal(host(out), want), pos
 
 
+@pytest.mark.parametrize("fused", [False, True])
+@pytest.mark.parametrize("max_seq", [200, 9000])  # PV and combine in one launch, and in two
+def test_attention_position_outside_the_caches(gpu, fused, max_seq):
+    """Positions the caches cannot hold: zeros, and no byte of the caches or the workspace, nor of what
+    lies behind them, is written."""
+    import torch
+    ident(f"attention position outside {max_seq} fused {fused}")
+    hq, hkv, D, behind = 4, 2, 128, 64
+    g = torch.Generator(device="cuda").manual_seed(max_seq)
+    x = [torch.randn(n, generator=g, device="cuda", dtype=torch.bfloat16)
+         for n in (hq * D, hkv * D, hkv * D, D, D)]
+    cache = torch.randn(2, max_seq + behind, hkv * D, generator=g, device="cuda", dtype=torch.bfloat16)
+    floats = gpu.attention_workspace_floats(hq, D, max_seq)
+    att = torch.randn(floats + behind * D * hq, generator=g, device="cuda")
+    held = [cache.clone(), att.clone()]
+    for pos in (max_seq, max_seq + 1, max_seq + 40, -1, -2, -200):
+        out = torch.ones(hq * D, device="cuda", dtype=torch.bfloat16)
+        if fused:
+            gpu.qk_norm_rope_attention_forward(out, *x, cache[0], cache[1], att, dev_i32([pos]), hq, hkv,
+                                               D, 1e-6, 1e6, max_seq, 0.1)
+        else:
+            gpu.attention_forward(out, x[0], cache[0], cache[1], att, hq, hkv, D, dev_i32([pos]), max_seq,
+                                  0.1)
+        torch.cuda.synchronize()
+        assert not out.any(), pos
+        assert torch.equal(cache, held[0]) and torch.equal(att, held[1]), pos
+
+
 # the shapes whose last blocks' workgroups are the most and the largest
 @pytest.mark.parametrize("hq,hkv,D,max_seq", [(64, 8, 128, 3072), (64, 8, 256, 1536), (64, 8, 128, 8192),
                                               (32, 8, 256, 3072)])
