@@ -1567,7 +1567,9 @@ __global__ __launch_bounds__(256) void attn_pv_kernel(AttnArgs a) {
 // columns of one query head (D / COMBINE_COLS workgroups per head, so the loads spread over
 // more CUs). The additions are sequential, the loads are not: the columns' partials are staged
 // in LDS by all 256 threads (every 16-byte load of a chunk of CB blocks in flight at once), then
-// thread c adds column c in block order, 16 LDS reads at a time.
+// thread c adds column c in block order, 16 LDS reads at a time, the next 16 in flight meanwhile (with
+// a test around each addition and no reads ahead, 32 heads on 8 of 128 at 8300 positions took 18.1 us
+// instead of 16.6, 1 on 1 of 64 at 16000 13.8 instead of 11.1).
 constexpr int COMBINE_COLS = 32;
 template <int D>
 __global__ __launch_bounds__(256) void attn_combine_kernel(AttnArgs a) {
@@ -1577,7 +1579,7 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnArgs a) {
     __shared__ float part[CB * CC];
     const int h = blockIdx.x / (D / CC), c0 = (blockIdx.x % (D / CC)) * CC;
     const float *src = a.partial + (size_t)h * a.max_blocks * D + c0;
-    float acc = 0.0f;
+    float acc = -0.0f;  // -0 + x is x, also for x = -0
     // Each chunk's loads cover min(CB, max_blocks - b0) blocks, whatever the history, and the
     // position is read after them (a per-lane load: as a uniform value it would be loaded, and
     // waited for, before them): one round trip instead of two. Blocks past the history are
@@ -1604,16 +1606,23 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(AttnArgs a) {
         const int cnt = min(CB, nb - b0);
         __syncthreads();
         if (threadIdx.x < CC) {
-            // 16 LDS reads in flight, then their additions in order
-            const int c = threadIdx.x;
-            for (int j0 = 0; j0 < cnt; j0 += 16) {
-                float v[16];
+            // in block order; 16 are added while the next 16 are read
+            const float *col = part + threadIdx.x;
+            const int whole = cnt & ~15;
+            float v[16], next[16];
 #pragma unroll
-                for (int j = 0; j < 16; j++) v[j] = part[min(j0 + j, cnt - 1) * CC + c];
+            for (int u = 0; u < 16; u++) v[u] = col[u * CC];
+            for (int j = 0; j < whole; j += 16) {
 #pragma unroll
-                for (int j = 0; j < 16; j++)
-                    if (j0 + j < cnt) acc = (b0 + j0 + j == 0) ? v[j] : acc + v[j];
+                for (int u = 0; u < 16; u++) next[u] = col[(min(j + 16, CB - 16) + u) * CC];
+#pragma unroll
+                for (int u = 0; u < 16; u++) acc += v[u];
+#pragma unroll
+                for (int u = 0; u < 16; u++) v[u] = next[u];
             }
+#pragma unroll
+            for (int u = 0; u < 15; u++)
+                if (whole + u < cnt) acc += v[u];
         }
     }
     if (threadIdx.x < CC) a.out[(size_t)h * D + c0 + threadIdx.x] = (bf16)f2bf(acc);
@@ -2163,20 +2172,21 @@ extern "C" void qk_norm_rope_attention_one_pass(bf16 *out, const bf16 *q, const 
 //
 // Bound by its chain (statistics, exponentials, the products, the count, the in-order sums) rather
 // than by the value stream, and at long histories by the one CU that reads a kv head's partials, at
-// some 50 GB/s. The line of PVC_MAX_FLOATS, from attention_forward of a full history in us, one launch
-// / two (heads on kv heads of head_dim, blocks):
-//   16 on 8 of 128: 8 blocks 7.6 / 8.5, 64 10.7 / 12.2, 128 14.6 / 15.7, 192 19.2 / 19.7, 256 30.5 / 23.2
-//   32 on 8 of 128: 8 7.6 / 9.2, 64 12.5 / 12.8, 128 17.1 / 17.3, 192 22.5 / 22.5, 256 33.9 / 26.4
-//   4 on 1 of 128: 8 8.0 / 8.6, 64 10.5 / 10.4, 96 12.3 / 11.3; 8 on 1: 16 10.3 / 11.0, 64 13.0 / 12.1
-//   64 on 8 of 256: 8 12.9 / 13.5, 16 14.2 / 14.2, 32 16.7 / 15.8; 1 on 1 of 64: 96 8.8 / 9.0, 128 10.2 / 9.7
-// The host knows the longest history only; shorter ones in the same caches gain most from one launch
-// (16 on 8 of 128 at 260 positions of 4096: 6.4 / 7.5), so the lines lie past the last full history
-// that gains. Past PVC_MAX_ITEMS the workgroups, which stay until their stores are acknowledged, no
-// longer fit the device at once (the 256-block figures of 8 kv heads).
+// some 50 GB/s. The lines, from attention_forward of a full history in us, one launch / two (heads on
+// kv heads of head_dim, blocks):
+//   16 on 8 of 128: 8 blocks 7.7 / 8.4, 64 10.8 / 11.5, 96 12.9 / 13.1, 128 15.2 / 14.7, 160 17.1 / 16.1
+//   32 on 8 of 128: 8 7.9 / 9.2, 48 11.2 / 11.3, 64 12.4 / 12.2, 96 14.8 / 14.2
+//   64 on 8 of 128: 8 10.1 / 11.1, 32 11.8 / 12.5, 48 14.2 / 14.3, 64 15.0 / 14.9
+//   64 on 8 of 256: 8 13.0 / 13.6, 16 14.1 / 14.5, 24 16.0 / 14.9
+//   1 on 1 of 64: 48 7.1 / 7.4, 64 7.9 / 7.9, 96 8.8 / 8.3; 8 on 8 of 64: 96 9.8 / 10.6, 128 11.1 / 11.3
+// The host knows the longest history only, and shorter ones in the same caches gain from one launch
+// (16 on 8 of 128 at 260 positions of 4096: 6.4 / 7.5). Past PVC_MAX_ITEMS the workgroups, which stay
+// until their stores are acknowledged, no longer fit the device at once: 16 on 16 of 128, 64 blocks
+// 12.2 / 13.4, 96 16.5 / 15.8, 128 24.9 / 18.6.
 // ------------------------------------------------------------------------------------------
 
-constexpr int PVC_MAX_FLOATS = 49152;  // partials of a kv head: blocks of the longest history x REP * D
-constexpr int PVC_MAX_BLOCKS = 128;
+constexpr int PVC_MAX_FLOATS = 32768;  // partials of a kv head: blocks of the longest history x REP * D
+constexpr int PVC_MAX_BLOCKS = 96;
 constexpr int PVC_MAX_ITEMS = 1280;    // blocks x kv heads
 static_assert(PVC_MAX_BLOCKS < 0x10000, "the count of a kv head's items fits 16 bits");
 

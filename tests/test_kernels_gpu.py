@@ -421,14 +421,16 @@ def test_attention_one_launch_combine(gpu, oracle, hq, hkv, D, pos, max_seq):
     assert np.array_equal(got, want)
 
 
-# histories around the combine's batches of blocks (32 columns' worth: 32, 16, 8 and 4 blocks at 64-256,
-# 512, 1024 and 2048 columns of a kv head), and the longest that one launch takes
+# histories around the combine's batches of blocks, and the longest that one launch takes; then two
+# launches, just past each limit and around the batches of 16 and 256 blocks
 @pytest.mark.parametrize("hq,hkv,D,max_seq,blocks", [
-    (2, 2, 64, 8192, (1, 31, 32, 33, 64, 65, 127, 128)), (16, 8, 128, 8192, (32, 33, 96, 97, 128)),
-    (2, 1, 256, 6144, (15, 16, 17, 32, 33, 96)), (4, 1, 256, 3072, (7, 8, 9, 16, 17, 47, 48)),
-    (16, 2, 256, 1536, (3, 4, 5, 8, 9, 24)), (16, 8, 128, 8193, (128, 129)), (16, 16, 64, 5121, (81,))])
+    (2, 2, 64, 6144, (1, 31, 32, 33, 64, 65, 95, 96)), (16, 8, 128, 6144, (32, 33, 64, 65, 96)),
+    (2, 1, 256, 4096, (15, 16, 17, 32, 33, 64)), (4, 1, 256, 2048, (7, 8, 9, 16, 17, 32)),
+    (16, 2, 256, 1024, (3, 4, 5, 8, 9, 16)),
+    (16, 8, 128, 6145, (96, 97)), (16, 2, 256, 1025, (16, 17)), (16, 16, 64, 5121, (80, 81)),
+    (2, 2, 64, 17408, (1, 15, 16, 17, 255, 256, 257, 272))])
 def test_attention_combine_batches(gpu, oracle, hq, hkv, D, max_seq, blocks):
-    """PV and combine in one launch, and in two just past its limits: bit-identical to the oracle at
+    """PV and combine in one launch and in two: bit-identical to the oracle at
     the first and the last position of each count of blocks, on one workspace that begins as ones."""
     import torch
     ident(f"attention combine batches {hq}/{hkv} D{D} of {max_seq}")
@@ -476,8 +478,8 @@ def test_attention_position_outside_the_caches(gpu, fused, max_seq):
 
 
 # the shapes whose last blocks' workgroups are the most and the largest
-@pytest.mark.parametrize("hq,hkv,D,max_seq", [(64, 8, 128, 3072), (64, 8, 256, 1536), (64, 8, 128, 8192),
-                                              (32, 8, 256, 3072)])
+@pytest.mark.parametrize("hq,hkv,D,max_seq", [(64, 8, 128, 2048), (64, 8, 256, 1024), (64, 8, 128, 8192),
+                                              (32, 8, 256, 2048)])
 def test_attention_overlapping_streams(gpu, hq, hkv, D, max_seq):
     """Attention calls of both forms on six streams at once, each with a workspace of its own: every
     result is that of the same call alone."""
