@@ -20,6 +20,9 @@ bool sample_step(int *out, const bf16 *x, int n, float inv_temp, float u, void *
 size_t sample_slot_bytes();
 // sample_forward draws from a row of n in one launch.
 bool sample_takes_one_launch(int n);
+// For tests, with no draw in flight: how many of the library's slots for sample_forward are taken (-1
+// after an error); then, with set 1 or 0, all are taken or free.
+extern "C" int llm_sample_slots(int set);
 
 // inv_freq_j = 1 / fp32(pow(theta, fp32(2j / D))) for j < D/2 (D <= 256), cached per (theta, D).
 void rope_inv_freq_table(float theta, int D, float *out);

@@ -10,8 +10,10 @@
 #include <stdarg.h>
 #include <string.h>
 
+#include <atomic>
 #include <mutex>
 #include <type_traits>
+#include <vector>
 
 #include "common.h"
 #include "internal.h"
@@ -2543,27 +2545,32 @@ extern "C" void attention_forward_noalloc(bf16 *out, const bf16 *q, const bf16 *
 //
 // Two launches for long rows: sample_kernel, one workgroup, takes the max (a row of 151936 is 300 KB,
 // read from L2); sample_sums_kernel spreads the weights, which are most of the work, over SAMPLE_WGS
-// workgroups, and the last of them to finish adds the chunk sums and draws. Between the two the chunk
-// sums live in one of SAMPLE_SLOTS library-owned slots, taken by the first launch with an atomic
-// exchange and given back by the second, so calls on any streams may overlap; `out` itself carries
-// the slot and the max from one launch to the next. With every slot taken the first launch draws
-// alone, as it does for rows of up to SAMPLE_ALONE.
+// workgroups, and the last of them to finish adds the chunk sums and draws. The chunk sums live in one
+// of SAMPLE_SLOTS library-owned slots. A call has a number, which both of its launches are given and
+// which names its slot: the first launch takes the slot and leaves the max in it, together with the
+// number, once for each workgroup of the second, which exchanges that word for a spent one before it
+// publishes. With the slot taken by another call the first launch draws alone, as it does for rows of up
+// to SAMPLE_ALONE, and the second finds no word of its number. So calls may overlap on any streams,
+// whatever they share. (Two launches of one captured graph at once have one number: one takes the slot,
+// the other draws alone, and whichever second launch comes first does the sums, the same ones.)
 //
-// Bound by its serial chains, which the order of the additions fixes (1024 dependent adds for the
-// total, about 150 per chunk), two launches and the round trips between them. 151936 logits: 105-119 us
-// on one workgroup, 19.6 us spread over 64, 17.0 us with the chains' LDS reads four deep, the max in the
-// ticket and the slot taken beside the max; 73.7 us on one workgroup now. The line at SAMPLE_ALONE: alone
-// 8.9 / 10.0 / 15.3 / 22.1 us at 4096 / 12288 / 16384 / 32768 logits, spread 13.2-13.5 us at each.
+// Bound by two launches and the round trips in and between them (the row's max by one workgroup, the
+// work's word, the sums' arrival, the sums, the drawn chunk's logits again): the additions whose order is
+// fixed, 1024 for the total and some 150 in each of two chunks, take 2.6 us at 4.6 clocks each. 151936
+// logits: 105-119 us on one workgroup, 19.6 us spread over 64, 17.5 us with the chains' LDS reads four
+// deep and the slot taken beside the max; 73.7 us on one workgroup now. The line at SAMPLE_ALONE: alone
+// 9.0 / 10.2 / 15.3 / 22.1 us at 4096 / 12288 / 16384 / 32768 logits, spread 13.4-13.8 us at each.
 constexpr int SAMPLE_T = 1024;
 constexpr int SAMPLE_WGS = 64, SAMPLE_ROWS = SAMPLE_T / SAMPLE_WGS;  // chunks per workgroup
 constexpr int SAMPLE_PIECE = 256;  // weights of a chunk staged at a time
-constexpr int SAMPLE_SLOTS = 16;
+constexpr int SAMPLE_SLOTS = 64;
 constexpr int SAMPLE_ALONE = 12288;  // longest row drawn in one launch
 
 struct SampleSlot {
     unsigned busy;   // taken by a call (of the library's slots)
     unsigned done;   // workgroups of the second launch that have published their sums
     float pad[30];
+    unsigned long long work[SAMPLE_WGS];  // of the library's: what workgroup w of the second launch does
     float sums[SAMPLE_T];
     float maxes[SAMPLE_WGS];  // of a step's slot: parts of the row's max
 };
@@ -2651,46 +2658,31 @@ __device__ __forceinline__ int sample_draw(const bf16 *x, int n, float inv_temp,
     return chosen;  // in the first wave
 }
 
-// What the first launch leaves in *out for the second: bit 31, the slot, and the row's max, which is
-// one of its bf16 values. (No drawn token looks like it: indexes have bit 31 clear, -1 has no slot.)
-__device__ __forceinline__ uint32_t sample_ticket(int slot, float mx) {
-    return 0x80000000u | (uint32_t)slot << 16 | __float_as_uint(mx) >> 16;
+// A word of SampleSlot::work: the call's number (40 bits, never 0), whether the work is still to be
+// done, and the row's max, which is one of its bf16 values.
+constexpr unsigned long long SAMPLE_OPEN = 1ull << 16;
+__host__ __device__ __forceinline__ unsigned long long sample_open_work(unsigned long long call) {
+    return call << 24 | SAMPLE_OPEN;
 }
 
-// The max of the row, then either the slot for sample_sums_kernel (spread != 0) or the whole draw.
+// The max of the row, then either the work of sample_sums_kernel (call != 0) or the whole draw.
 // The last wave takes the slot before it reads its part of the row. vec: x is 16-byte aligned.
 __global__ __launch_bounds__(SAMPLE_T) void sample_kernel(int *out, const bf16 *x, int n,
                                                           float inv_temp, float u, int vec,
-                                                          int spread) {
+                                                          unsigned long long call) {
     __shared__ __align__(16) float sums[SAMPLE_T];
     __shared__ __align__(16) float piece[SAMPLE_PIECE];
     __shared__ float wmax[SAMPLE_T / 64];
     __shared__ float share[3];
-    __shared__ int s_slot;
+    __shared__ int s_taken;
     const int t = threadIdx.x;
-    if (spread && wave_id() == SAMPLE_T / 64 - 1) {
-        // lanes 0 .. SAMPLE_SLOTS - 1 look at one slot each, the lowest free one is taken
-        const int lane = t & 63;
-        int slot = -1;
-        const bool free = lane < SAMPLE_SLOTS &&
-                          __hip_atomic_load(gptr(&g_sample_slots[lane & (SAMPLE_SLOTS - 1)].busy),
-                                            __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
-        unsigned long long left = __ballot(free);
-        while (left && slot < 0) {
-            const int s = __ffsll(left) - 1;
-            left &= left - 1;
-            unsigned was = 1;
-            if (lane == 0)
-                was = __hip_atomic_exchange(gptr(&g_sample_slots[s].busy), 1u, __ATOMIC_RELAXED,
-                                            __HIP_MEMORY_SCOPE_AGENT);
-            if (__builtin_amdgcn_readfirstlane(was) == 0) slot = s;
-        }
-        if (lane == 0) {
-            s_slot = slot;
-            if (slot >= 0)
-                __hip_atomic_store(gptr(&g_sample_slots[slot].done), 0u, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-        }
+    SampleSlot &sl = g_sample_slots[call % SAMPLE_SLOTS];
+    if (call && t == SAMPLE_T - 64) {
+        s_taken = __hip_atomic_exchange(gptr(&sl.busy), 1u, __ATOMIC_RELAXED,
+                                        __HIP_MEMORY_SCOPE_AGENT) == 0;
+        if (s_taken)
+            __hip_atomic_store(gptr(&sl.done), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // before any work is open
     }
     float m = -__builtin_huge_valf();
     int done = 0;
@@ -2716,8 +2708,10 @@ __global__ __launch_bounds__(SAMPLE_T) void sample_kernel(int *out, const bf16 *
     float mx = wmax[0];
 #pragma unroll
     for (int w = 1; w < SAMPLE_T / 64; w++) mx = fmaxf(mx, wmax[w]);  // max: any order
-    if (spread && s_slot >= 0) {
-        if (t == 0) *out = (int)sample_ticket(s_slot, mx);
+    if (call && s_taken) {
+        if (t < SAMPLE_WGS)
+            __hip_atomic_store(gptr(&sl.work[t]), sample_open_work(call) | __float_as_uint(mx) >> 16,
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return;
     }
     const int chunk = (n + SAMPLE_T - 1) / SAMPLE_T;
@@ -2731,12 +2725,13 @@ __global__ __launch_bounds__(SAMPLE_T) void sample_kernel(int *out, const bf16 *
 }
 
 // A decode step draws with a slot of its own, in which sample_max_kernel has left the row's max in
-// parts (traced in a sampled 4B decode: 4.5 us, against 5.6 with one workgroup). The drawn token is also handed to the host, with the
-// step's error flag, in the two pinned words at mail.
+// parts (traced in a sampled 4B decode: 4.5 us, against 5.6 with one workgroup). The drawn token is
+// also handed to the host, with the step's error flag, in the two pinned words at mail.
 struct SampleStep {
-    SampleSlot *slot;  // NULL: the slot and the max are in the ticket
+    SampleSlot *slot;  // NULL: the library's slot of the call
     int *mail;
     const int *err;
+    unsigned long long call;
 };
 
 // Workgroup w's part of the row's max. vec: x is 16-byte aligned.
@@ -2768,6 +2763,7 @@ __global__ __launch_bounds__(256) void sample_sums_kernel(int *out, const bf16 *
     __shared__ __align__(16) float stage[R * (P + 1)];  // padded rows: lanes 0..R-1 read one column
     __shared__ float share[3];
     __shared__ int s_last;
+    __shared__ unsigned long long s_work;
     static_assert(R * (P + 1) >= SAMPLE_T + P, "the draw reuses the staging");
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     const int chunk = (n + SAMPLE_T - 1) / SAMPLE_T;
@@ -2784,20 +2780,27 @@ __global__ __launch_bounds__(256) void sample_sums_kernel(int *out, const bf16 *
                 v[r][j] = x[min(at, (long long)n - 1)];
             }
     };
-    request(0);  // before the wait for the ticket
-    const uint32_t ticket = (uint32_t)*out;
-    SampleSlot *slot = step.slot;
+    request(0);  // before the wait for the max
+    SampleSlot &sl = step.slot ? *step.slot : g_sample_slots[step.call % SAMPLE_SLOTS];
     float mx;
+    bool mine = true;  // (of the first wave) its sums are the ones to publish
     static_assert(SAMPLE_WGS == 64, "a lane per part");
-    if (slot) {
-        mx = wave_max(slot->maxes[lane]);
+    if (step.slot) {
+        mx = wave_max(sl.maxes[lane]);
     } else {
-        // not a ticket: the first launch has drawn
-        if (!(ticket >> 31) || (ticket >> 16 & 0x7fff) >= SAMPLE_SLOTS) return;
-        slot = &g_sample_slots[ticket >> 16 & 0x7fff];
-        mx = __uint_as_float(ticket << 16);
+        if (t == 0)
+            s_work = __hip_atomic_load(gptr(&sl.work[blockIdx.x]), __ATOMIC_RELAXED,
+                                       __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        unsigned long long word = s_work;
+        // the first launch has drawn, or this work is done
+        if (word >> 16 != sample_open_work(step.call) >> 16) return;
+        mx = __uint_as_float((uint32_t)word << 16);
+        if (t == 0)
+            mine = __hip_atomic_compare_exchange_strong(gptr(&sl.work[blockIdx.x]), &word,
+                                                        word ^ SAMPLE_OPEN, __ATOMIC_RELAXED,
+                                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-    SampleSlot &sl = *slot;
     float acc = 0.0f;
     for (int b = 0; b < chunk; b += P) {
         const int len = min(P, chunk - b);
@@ -2837,14 +2840,15 @@ __global__ __launch_bounds__(256) void sample_sums_kernel(int *out, const bf16 *
         }
         __syncthreads();
     }
-    if (t < R)
+    if (w == 0) mine = __builtin_amdgcn_readfirstlane(mine);
+    if (t < R && mine)
         __hip_atomic_store(gptr(&sl.sums[k0 + t]), acc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     // The sums are written through to the level all XCDs share, by this wave alone: once they are
     // acknowledged there, the arrival needs no release of its own (which writes back the whole L2).
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (t == 0)
-        s_last = __hip_atomic_fetch_add(gptr(&sl.done), 1u, __ATOMIC_RELAXED,
-                                        __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+        s_last = mine && __hip_atomic_fetch_add(gptr(&sl.done), 1u, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
     __syncthreads();
     if (!s_last) return;
     float *sums = stage, *piece = stage + SAMPLE_T;
@@ -2872,17 +2876,46 @@ __global__ __launch_bounds__(256) void sample_sums_kernel(int *out, const bf16 *
     }
 }
 
+// Gives back the slot that call's first launch has taken, where the second could not be launched.
+__global__ __launch_bounds__(SAMPLE_WGS) void sample_give_back_kernel(unsigned long long call) {
+    SampleSlot &sl = g_sample_slots[call % SAMPLE_SLOTS];
+    unsigned long long word = sl.work[threadIdx.x];
+    const bool closed =
+        word >> 16 == sample_open_work(call) >> 16 &&
+        __hip_atomic_compare_exchange_strong(gptr(&sl.work[threadIdx.x]), &word, word ^ SAMPLE_OPEN,
+                                             __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                             __HIP_MEMORY_SCOPE_AGENT);
+    if (__ballot(closed) == ~0ull && threadIdx.x == 0)
+        __hip_atomic_store(gptr(&sl.busy), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 extern "C" void sample_forward(int *out, const bf16 *x, int n, float inv_temp, float u,
                                hipStream_t stream) {
     if (n <= 0) {
         llm_fail("sample: n %d must be positive", n);
         return;
     }
-    const int spread = n > SAMPLE_ALONE;
-    sample_kernel<<<1, SAMPLE_T, 0, stream>>>(out, x, n, inv_temp, u, aligned16(x) ? 1 : 0, spread);
-    if (!LAUNCH_OK() || !spread) return;
-    sample_sums_kernel<<<SAMPLE_WGS, 256, 0, stream>>>(out, x, n, inv_temp, u, SampleStep{});
-    LAUNCH_OK();
+    static std::atomic<unsigned long long> calls;
+    const unsigned long long call =
+        n > SAMPLE_ALONE ? 1 + calls.fetch_add(1, std::memory_order_relaxed) % ((1ull << 40) - 1) : 0;
+    sample_kernel<<<1, SAMPLE_T, 0, stream>>>(out, x, n, inv_temp, u, aligned16(x) ? 1 : 0, call);
+    if (!LAUNCH_OK() || !call) return;
+    sample_sums_kernel<<<SAMPLE_WGS, 256, 0, stream>>>(out, x, n, inv_temp, u,
+                                                       SampleStep{nullptr, nullptr, nullptr, call});
+    if (!LAUNCH_OK()) sample_give_back_kernel<<<1, SAMPLE_WGS, 0, stream>>>(call);
+}
+
+extern "C" int llm_sample_slots(int set) {
+    std::vector<SampleSlot> slots(SAMPLE_SLOTS);
+    int taken = 0;
+    const size_t bytes = sizeof(SampleSlot) * SAMPLE_SLOTS;
+    if (!HIP_OK(hipMemcpyFromSymbol(slots.data(), HIP_SYMBOL(g_sample_slots), bytes))) return -1;
+    for (SampleSlot &slot : slots) {
+        taken += slot.busy != 0;
+        if (set >= 0) slot.busy = (unsigned)set;
+    }
+    if (set >= 0 && !HIP_OK(hipMemcpyToSymbol(HIP_SYMBOL(g_sample_slots), slots.data(), bytes))) return -1;
+    return taken;
 }
 
 size_t sample_slot_bytes() { return sizeof(SampleSlot); }
@@ -2893,7 +2926,7 @@ bool sample_step(int *out, const bf16 *x, int n, float inv_temp, float u, void *
     sample_max_kernel<<<SAMPLE_WGS, 256, 0, stream>>>((SampleSlot *)slot, x, n, aligned16(x) ? 1 : 0);
     if (!LAUNCH_OK()) return false;
     sample_sums_kernel<<<SAMPLE_WGS, 256, 0, stream>>>(out, x, n, inv_temp, u,
-                                                       SampleStep{(SampleSlot *)slot, mail, err});
+                                                       SampleStep{(SampleSlot *)slot, mail, err, 0});
     return LAUNCH_OK();
 }
 

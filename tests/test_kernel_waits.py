@@ -40,3 +40,12 @@ def test_only_the_one_pass_attention_waits():
     assert waits & kernels == {"attn_one_pass_kernel"}
     contract = (ROOT / "include" / "llm_amd" / "kernels.h").read_text()
     assert re.search(r"workgroups wait for each\s+\*\s+other", contract)
+
+
+def test_the_draw_keeps_nothing_in_out():
+    """`out` belongs to the caller, who may give the same one to overlapping calls: no kernel of
+    sample_forward reads it."""
+    bodies = functions((PKG_DIR / "csrc" / "kernels.hip").read_text())
+    for name in ("sample_kernel", "sample_sums_kernel"):
+        uses = re.findall(r"[^;{}]*\bout\b[^;{}]*", bodies[name])
+        assert uses and all(re.fullmatch(r"\s*(if \(t == 0\)\s*)?\*out = chosen", u) for u in uses), uses

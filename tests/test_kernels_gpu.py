@@ -912,6 +912,91 @@ def test_sample_forward_overlapping_streams_and_graph(gpu, oracle):
         assert outs.cpu().tolist() == want
 
 
+@pytest.mark.parametrize("n", [12289, 151936])
+def test_sample_forward_with_every_slot_taken(gpu, oracle, n):
+    """A call that finds its slot taken draws in its first launch; slots given back serve again."""
+    import torch
+    ident(f"sample_forward without slots, row of {n}")
+    rng = np.random.default_rng(n)
+    row = rand_bf16(rng, n, 2.0)
+    xd, out = dev(row), torch.zeros(1, dtype=torch.int32, device="cuda")
+    coins = [float(c) for c in rng.random(4)]
+    want = [oracle.sample(row, 0.8, c) for c in coins]
+    for taken in (1, 0):
+        torch.cuda.synchronize()
+        assert gpu.lib().llm_sample_slots(taken) == 0
+        for c, w in zip(coins, want):
+            gpu.sample_forward(out, xd, n, 0.8, c)
+            assert int(out.item()) == w
+        assert gpu.lib().llm_sample_slots(0) == (64 if taken else 0)
+
+
+def test_sample_forward_shared_out(gpu, oracle):
+    """Overlapping calls that share `out`, on rows of their own: it ends with the token of one of them,
+    other callers draw theirs, and no slot stays taken."""
+    import torch
+    ident("sample_forward with a shared out")
+    rng = np.random.default_rng(78)
+    n = 151936
+    rows = [rand_bf16(rng, n, 2.0) for _ in range(4)]
+    xs = [dev(r) for r in rows]
+    want = [oracle.sample(r, 0.8, 0.5) for r in rows]
+    streams = [torch.cuda.Stream() for _ in rows]
+    shared, own = (torch.zeros(k, dtype=torch.int32, device="cuda") for k in (1, 40))
+    torch.cuda.synchronize()
+    for i in range(40):
+        for x, s in zip(xs[:3], streams):
+            gpu.sample_forward(shared, x, n, 0.8, 0.5, stream=s)
+        gpu.sample_forward(own[i:], xs[3], n, 0.8, 0.5, stream=streams[3])
+    torch.cuda.synchronize()
+    assert int(shared.item()) in want[:3]
+    assert own.tolist() == [want[3]] * 40
+    assert gpu.lib().llm_sample_slots(-1) == 0
+
+
+def test_sample_forward_two_instances_of_a_graph(gpu, oracle):
+    """One captured draw, instantiated twice and launched on two streams at once, with eager draws
+    beside it: both instances have the same inputs and the same `out`, and give the same token."""
+    import ctypes
+    import torch
+    from llm_inference_amd import model
+    ident("sample_forward in two instances of a graph")
+    rt = model._hip()
+    rng = np.random.default_rng(79)
+    n = 151936
+    rows = [rand_bf16(rng, n, 2.0) for _ in range(2)]
+    xs = [dev(r) for r in rows]
+    want = [oracle.sample(r, 0.8, 0.5) for r in rows]
+    out, eager = (torch.zeros(k, dtype=torch.int32, device="cuda") for k in (1, 30))
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(streams[0]):
+        graph.capture_begin()
+        gpu.sample_forward(out, xs[0], n, 0.8, 0.5)
+        graph.capture_end()
+    execs = [ctypes.c_void_p() for _ in range(2)]
+    raw = ctypes.c_void_p(graph.raw_cuda_graph())
+    for e in execs:
+        assert rt.hipGraphInstantiate(ctypes.byref(e), raw, None, None, ctypes.c_size_t(0)) == 0
+    try:
+        for i in range(30):
+            out.fill_(-7)
+            torch.cuda.synchronize()
+            for _ in range(3):
+                for e, s in zip(execs, streams):
+                    assert rt.hipGraphLaunch(e, ctypes.c_void_p(s.cuda_stream)) == 0
+            gpu.sample_forward(eager[i:], xs[1], n, 0.8, 0.5, stream=streams[2])
+            torch.cuda.synchronize()
+            assert int(out.item()) == want[0]
+        assert eager.tolist() == [want[1]] * 30
+        assert gpu.lib().llm_sample_slots(-1) == 0
+    finally:
+        torch.cuda.synchronize()
+        for e in execs:
+            rt.hipGraphExecDestroy(e)
+
+
 # ---------------------------------------------------------------- argmax
 
 def test_argmax(gpu, oracle):
