@@ -5,17 +5,22 @@ replaces the reference's src/kernels.cuh and src/forward.cuh launchers and step 
 (William-Lamer/llm-inference). The wrappers take torch tensors for device memory and a torch
 stream (or the current one); torch is only the allocator and stream provider. Every call goes to
 the HIP kernels: there is no CPU path, and a missing library raises. The launchers are called
-through a native module (csrc/launchers.cpp), arguments it does not recognise through ctypes.
+through a native module (csrc/launchers.cpp) where one is built for this Python and torch, and
+through ctypes otherwise and for arguments that it does not recognise.
 
 Errors the reference reports with exit(EXIT_FAILURE) raise LlmError here (the library is
 switched to recording mode on load).
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 from pathlib import Path
 
 HERE = Path(__file__).resolve().parent
 LIB_PATH = HERE / "libllm_amd.so"
+# the module built for this very Python (another's is not looked at)
+LAUNCHERS_PATH = HERE / ("_launchers" + importlib.machinery.EXTENSION_SUFFIXES[0])
 
 __all__ = [
     "LlmError", "lib", "embedding_forward", "rmsnorm_forward", "gemv_forward",
@@ -51,7 +56,7 @@ class LlmError(RuntimeError):
 
 
 _lib = None
-_native = None  # the _launchers module, once the library is loaded
+_native = None  # the launchers' module, once the library is loaded; None: every call through ctypes
 
 _vp = ctypes.c_void_p
 _i = ctypes.c_int
@@ -94,13 +99,29 @@ _SIGS = {
 }
 
 
+def _load_launchers(torch_version):
+    """The native launchers, or None where none are built for this Python and torch: their every call
+    goes through ctypes as well, with more host time."""
+    try:
+        name = __name__ + "._launchers"
+        loader = importlib.machinery.ExtensionFileLoader(name, str(LAUNCHERS_PATH))
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader(name, loader))
+        loader.exec_module(module)
+    except ImportError:
+        return None
+    if module.TORCH_VERSION != torch_version.split("+")[0]:
+        return None
+    module.init(LlmError)
+    return module
+
+
 def lib():
     """The loaded libllm_amd.so (raises LlmError if it has not been built)."""
     global _lib, _native
     if _lib is None:
         # torch first: its bundled HIP runtime then satisfies the library's libamdhip64.so.7
         # dependency (same SONAME), so both share one runtime and torch's streams are valid here.
-        import torch  # noqa: F401
+        import torch
         if not LIB_PATH.exists():
             raise LlmError(f"{LIB_PATH} is missing: build it with `make -C {HERE}` "
                            "(or __graft_entry__.build())")
@@ -110,13 +131,7 @@ def lib():
             fn.restype = res
             fn.argtypes = args
         L.llm_set_exit_on_error(0)
-        try:
-            from . import _launchers
-        except ImportError as e:
-            raise LlmError(f"{HERE / '_launchers.so'} is missing or does not load ({e}): build it "
-                           f"with `make -C {HERE}` (or __graft_entry__.build())") from e
-        _launchers.init(LlmError)
-        _lib, _native = L, _launchers
+        _lib, _native = L, _load_launchers(torch.__version__)
         from . import model  # noqa: F401  (declares the step API signatures)
         model._declare(L)
     return _lib

@@ -17,6 +17,7 @@
 
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/version.h>
 
 #include <limits.h>
 #include <stddef.h>
@@ -194,4 +195,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_launchers", nullptr, -1, methods}
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__launchers(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__launchers(void) {
+    PyObject *m = PyModule_Create(&module);
+    // the torch whose tensors this reads: the package leaves the module alone under another
+    if (m && PyModule_AddStringConstant(m, "TORCH_VERSION", TORCH_VERSION) < 0) Py_CLEAR(m);
+    return m;
+}

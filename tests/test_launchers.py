@@ -1,11 +1,13 @@
 """The native launchers (csrc/launchers.cpp) against the general ctypes way of the same wrappers:
 every form of argument gives the same result, or the same error."""
 import math
+import subprocess
+import sys
 
 import numpy as np
 import pytest
 
-from conftest import rand_bf16
+from conftest import PKG_DIR, ROOT, rand_bf16
 
 
 def outcome(fn, *args, **kw):
@@ -23,6 +25,37 @@ def both(pkg, monkeypatch, name, *args, **kw):
         m.setattr(pkg, "_native", None)
         general = outcome(getattr(pkg, name), *args, **kw)
     return native, general
+
+
+def test_built_for_this_python(pkg):
+    pkg.lib()
+    assert pkg._native is not None and pkg._native.__file__ == str(pkg.LAUNCHERS_PATH)
+
+
+@pytest.mark.parametrize("setup", [
+    "pkg.LAUNCHERS_PATH = pathlib.Path('/nonexistent/_launchers.so')",
+    "pkg.LAUNCHERS_PATH = pathlib.Path(pkg.__file__)",  # no shared object
+    "pkg.LAUNCHERS_PATH = pkg.HERE.parent / 'oracle' / 'liboracle.so'",  # no module
+    "import torch; torch.__version__ = '0.0.0'"])
+def test_the_library_works_without_them(setup):
+    """A module that is missing, does not load or was built over another torch: every call goes
+    through ctypes."""
+    code = ("import pathlib, sys; sys.path.insert(0, 'tests'); from conftest import load_package;"
+            f"pkg = load_package(); {setup}; pkg.lib(); assert pkg._native is None\n"
+            "try: pkg.gemv_forward(4096, 4096, 4096, 4, 7, stream=0)\n"
+            "except pkg.LlmError as e: print(e)")
+    r = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True, check=True)
+    assert "cols 7 is not a multiple of 8" in r.stdout
+
+
+@pytest.mark.parametrize("lacking", ["PY_INC=/nonexistent", "TORCH=/nonexistent", "PYTHON=/nonexistent"])
+def test_make_builds_the_library_without_headers_or_torch(lacking):
+    def plan(*args):
+        return subprocess.run(["make", "-n", "-B", "-C", str(PKG_DIR), *args], capture_output=True,
+                              text=True, check=True).stdout
+    assert "launchers.cpp" in plan(f"PYTHON={sys.executable}")
+    lean = plan(lacking)
+    assert "launchers.cpp" not in lean and "libllm_amd.so" in lean
 
 
 # calls that the library or the wrapper refuses before a launch: no GPU needed
