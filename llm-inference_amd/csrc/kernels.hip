@@ -166,8 +166,11 @@ __global__ __launch_bounds__(256) void rmsnorm_wave_kernel(bf16 *out, const bf16
 // Bound by memory: 16-byte accesses at whatever element the row begins (rows of odd dims cross more
 // cache lines than those that begin on a multiple of 4 or 16 bytes). The element-by-element form it
 // replaces read each row twice with a bounds test per element: 1000 x 9000 31.0 -> 7.4 us (4.9 TB/s),
-// 1000 x 9001 32.2 -> 9.2, 4096 x 8190 80.3 -> 27.5, 4096 x 2561 26.9 -> 10.5, 1 x 9000 16.8 -> 3.4,
-// 4096 x 101 3.9 -> 3.8. Up to two chunks per thread the stores are plain: such rows end inside cache
+// 1000 x 9001 32.2 -> 9.2, 1000 x 30000 71.9 -> 24.9, 4096 x 8190 80.3 -> 27.5, 4096 x 2561 26.9 -> 10.5,
+// 1 x 9000 16.8 -> 3.4, 4096 x 101 3.9 -> 3.8. Over 32768 wide a row takes 5 to 16 waves, whose 128
+// registers a thread do not hold 16 chunks and the arithmetic: 26 of them go to scratch (108 bytes a
+// thread), still 1000 x 32769 65.9 -> 45.3, 1000 x 40000 83.9 -> 38.6, 1000 x 65536 108 -> 57.5,
+// 500 x 131072 110 -> 62.7. Up to two chunks per thread the stores are plain: such rows end inside cache
 // lines that others begin in (4096 x 101 4.2 us with non-temporal ones, 4096 x 1025 5.7 against 5.5;
 // 1000 x 9000 8.4 with plain ones).
 template <int NC, int THREADS>
@@ -234,7 +237,7 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_rows_kernel(bf16 *out, const 
     if (tail) store(dim - 8, xl, wl);  // over elements of the last chunk too: the same values
 }
 
-// The rest (dim < 8, or over 16 chunks per thread: dim > 131072): the same sums, element by element.
+// The rest (dim < 8, or over 16 chunks per thread: dim > 131079): the same sums, element by element.
 __global__ __launch_bounds__(1024) void rmsnorm_generic_kernel(bf16 *out, const bf16 *in,
                                                                const bf16 *weight, int dim,
                                                                float eps) {
@@ -3119,7 +3122,8 @@ __device__ __forceinline__ void block_amax(float &v, int &i, float *lv, int *li)
 }
 
 // A row that one workgroup reads in less time than a second launch takes. Each thread sees its elements
-// in ascending order, so a strict comparison keeps the lowest index of its largest value.
+// in ascending order, so its largest value keeps the lowest index (the comparison of equal values by
+// index lets the first -inf in, which equals the value a thread begins with).
 //
 // Bound by its launch and its round trips. One launch here / two launches: 2.8 / 4.4 us at 1000 values,
 // 3.5 / 4.8 at 8192, 4.6 / 4.9 at 24576, 5.2 / 4.9 at 32768.
