@@ -20,6 +20,9 @@ bool sample_step(int *out, const bf16 *x, int n, float inv_temp, float u, void *
 size_t sample_slot_bytes();
 // sample_forward draws from a row of n in one launch.
 bool sample_takes_one_launch(int n);
+// For tests: out[i] = exp_f32 (branches: the form with early returns) of the float with the bits
+// first + i, i < n.
+extern "C" void llm_exp_bits(float *out, unsigned first, unsigned n, int branches, hipStream_t stream);
 // For tests, with no draw in flight: how many of the library's slots for sample_forward are taken (-1
 // after an error); then, with set 1 or 0, all are taken or free.
 extern "C" int llm_sample_slots(int set);

@@ -2933,6 +2933,19 @@ bool sample_step(int *out, const bf16 *x, int n, float inv_temp, float u, void *
     return LAUNCH_OK();
 }
 
+__global__ __launch_bounds__(256) void exp_bits_kernel(float *out, unsigned first, unsigned n,
+                                                       int branches) {
+    for (size_t i = blockIdx.x * (size_t)256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
+        const float x = __uint_as_float(first + (unsigned)i);
+        out[i] = branches ? exp_f32<true>(x) : exp_f32(x);
+    }
+}
+
+extern "C" void llm_exp_bits(float *out, unsigned first, unsigned n, int branches, hipStream_t stream) {
+    exp_bits_kernel<<<4096, 256, 0, stream>>>(out, first, n, branches);
+    LAUNCH_OK();
+}
+
 // ------------------------------------------------------------------------------------------
 // streaming ceiling probe (measurement helper)
 // ------------------------------------------------------------------------------------------

@@ -69,7 +69,7 @@ def test_rmsnorm(gpu, oracle, rows, dim):
 
 
 # one chunk and a tail, the last whole chunk of a wave, one to two waves (8192), two to five, the
-# widest held in registers (131079) and the next row that is not; element offsets of the buffers
+# widest in chunks (131079) and the next row that is not; element offsets of the buffers
 @pytest.mark.parametrize("dim", [7, 9, 15, 511, 513, 1023, 5000, 8191, 8193, 8200, 9001, 16384, 16391,
                                  32773, 131079, 131080])
 @pytest.mark.parametrize("offset", [0, 1, 4])
@@ -836,6 +836,39 @@ def test_hbm_copy_peak_probe(gpu):
         gpu.hbm_copy_peak_probe(d, a, 24, 4, 256)
     with pytest.raises(gpu.LlmError):
         gpu.hbm_copy_peak_probe(d, a, 64, 4, 256, 3)
+
+
+# ---------------------------------------------------------------- exponential
+
+def test_exp_forms_agree_for_every_float(gpu, oracle):
+    """The device's exponential without branches and with early returns: the same bits for each of the
+    2^32 fp32 inputs (both zeros, infinities, denormals and every NaN among them), and the oracle's on
+    a sample of them and around the limits of the clamp and the early returns."""
+    import ctypes
+    import torch
+    ident("exp_f32 over every fp32 input")
+    fn = gpu.lib().llm_exp_bits
+    fn.argtypes = [ctypes.c_void_p, ctypes.c_uint32, ctypes.c_uint32, ctypes.c_int, ctypes.c_void_p]
+    fn.restype = None
+    stream = torch.cuda.current_stream().cuda_stream
+    chunk = 1 << 28
+    a, b = (torch.empty(chunk, dtype=torch.int32, device="cuda") for _ in range(2))
+    rng = np.random.default_rng(104)
+    edges = np.float32([-105, -104, -103.97, -87.3, 0, 88.72, 88.73, 89, 90, np.inf, -np.inf])
+    edges = (edges.view(np.uint32)[:, None].astype(np.int64) + np.arange(-40, 41)).reshape(-1)
+    bits = np.unique(np.concatenate([edges, rng.integers(0, 1 << 32, 20000)]) & 0xFFFFFFFF)
+    for first in range(0, 1 << 32, chunk):
+        for t, branches in ((a, 0), (b, 1)):
+            fn(t.data_ptr(), first, chunk, branches, stream)
+        assert torch.equal(a, b), hex(first)
+        some = bits[(bits >= first) & (bits < first + chunk)]
+        got = a[torch.from_numpy(some - first).cuda()].cpu().numpy().view(np.float32)
+        x = some.astype(np.uint32).view(np.float32)
+        want = np.float32([oracle.exp_f32(v) for v in x])
+        nan = np.isnan(x)
+        assert np.array_equal(got.view(np.uint32)[~nan], want.view(np.uint32)[~nan])
+        assert np.isnan(got[nan]).all()
+    gpu.check()
 
 
 # ---------------------------------------------------------------- temperature sampling

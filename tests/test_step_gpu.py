@@ -1004,6 +1004,47 @@ def test_persistent_step_wide_shapes_long_history(gpu, oracle, size):
         dec.close()
 
 
+@pytest.mark.parametrize("size,switch", [("1.7B", 4480), ("4B", 4096)])
+def test_auto_step_switches_wide_shapes(gpu, oracle, size, switch):
+    """STEP_AUTO's switch from the persistent kernel to the hipGraph at the 1.7B and 4B widths (2 layers,
+    caches filled with N(0, 1)): single steps on both sides of it, with logits and argmax bit-identical
+    to the oracle and a sampled token each, and one generate_greedy call across it."""
+    ident(f"auto step switch at {size} widths")
+    from llm_inference_amd import model
+    S = switch + 24
+    cfg = model.qwen3_config(size, n_layers=2, max_seq_len=S)
+    dec = model.Decoder(cfg, ("synth", 32, 0.02, 0.1))
+    try:
+        rng = np.random.default_rng(switch)
+        kvd = cfg.n_kv_heads * cfg.head_dim
+        k = rand_bf16(rng, (cfg.n_layers, S, kvd))
+        v = rand_bf16(rng, (cfg.n_layers, S, kvd))
+        dec.set_kv_cache(k, v)
+        w = dec.host_weights()
+        orc = oracle.Model(oracle_cfg(cfg), w, max_seq=S)
+        del w
+        orc.bufs["key_cache"][:] = k.reshape(-1)
+        orc.bufs["value_cache"][:] = v.reshape(-1)
+        dec.capture_graph("auto")
+        assert dec.persistent and dec.s.step_switch_pos == switch
+        assert dec.kernel_tokens(switch - 6, 12) == 6
+        got, t, want = dec.generate_greedy(77, switch - 6, 12), 77, []
+        for i in range(12):
+            t = orc.forward(t, switch - 6 + i, oracle.GPU_ORDER)
+            want.append(t)
+        assert got == want
+        for pos in (switch - 1, switch, switch + 20):
+            tok = int(rng.integers(0, cfg.vocab_size))
+            dec.forward(tok, pos)
+            ref = orc.forward(tok, pos, oracle.GPU_ORDER)
+            assert np.array_equal(dec.logits(), orc.logits), pos
+            drawn = oracle.sample(orc.logits, float(np.float32(1) / np.float32(0.8)), 0.37)
+            assert dec.sample_temperature(0.8, 0.37) == drawn
+            assert dec.sample_argmax() == ref, pos
+    finally:
+        dec.close()
+
+
 @pytest.mark.parametrize("mode", ["graph", "persistent"])
 def test_step_keeps_an_earlier_error_code(gpu, mode):
     """A wait between workgroups that finds the error flag already set stops at once and leaves
