@@ -1407,7 +1407,9 @@ __device__ __forceinline__ void pv_item(const AttnArgs &a, int b, int g, int n, 
                                         float (&p_s)[REP][ATT_B], float (&red)[4][REP][D],
                                         Store store) {
     constexpr int LP = D / 8, PPW = 64 / LP, PER_WAVE = ATT_B / 4, ITERS = PER_WAVE / PPW;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    // not held over attn_pv_kernel's items, in which they took up to 15 registers: a PV pass of its own is
+    // 0.1 to 0.6 us shorter (8 heads on 8 of 256 at 4000 positions 13.1 -> 12.5 an attention_forward)
+    const int lane = tid_x() & 63, w = wave_id();
     const int G = lane / LP, L = lane % LP;
     const int kv_dim = a.n_kv_heads * D;
     // The first head of this wave (r = w, where it has one): its score and block statistics are
@@ -2179,15 +2181,15 @@ extern "C" void qk_norm_rope_attention_one_pass(bf16 *out, const bf16 *q, const 
 // than by the value stream, and at long histories by the one CU that reads a kv head's partials, at
 // some 50 GB/s. The lines, from attention_forward of a full history in us, one launch / two (heads on
 // kv heads of head_dim, blocks):
-//   16 on 8 of 128: 8 blocks 7.7 / 8.4, 64 10.8 / 11.5, 96 12.9 / 13.1, 128 15.2 / 14.7, 160 17.1 / 16.1
-//   32 on 8 of 128: 8 7.9 / 9.2, 48 11.2 / 11.3, 64 12.4 / 12.2, 96 14.8 / 14.2
-//   64 on 8 of 128: 8 10.1 / 11.1, 32 11.8 / 12.5, 48 14.2 / 14.3, 64 15.0 / 14.9
-//   64 on 8 of 256: 8 13.0 / 13.6, 16 14.1 / 14.5, 24 16.0 / 14.9
-//   1 on 1 of 64: 48 7.1 / 7.4, 64 7.9 / 7.9, 96 8.8 / 8.3; 8 on 8 of 64: 96 9.8 / 10.6, 128 11.1 / 11.3
+//   16 on 8 of 128: 8 blocks 7.8 / 8.2, 64 10.9 / 11.1, 96 12.9 / 12.8, 128 15.1 / 14.5, 160 17.0 / 15.9
+//   32 on 8 of 128: 8 7.8 / 8.8, 48 11.2 / 11.2, 64 12.4 / 11.9, 96 14.8 / 13.8
+//   64 on 8 of 128: 8 9.9 / 11.1, 32 11.9 / 12.6, 48 14.2 / 14.3, 64 15.0 / 14.8
+//   64 on 8 of 256: 8 13.1 / 13.6, 16 14.1 / 14.3, 24 16.1 / 14.7
+//   1 on 1 of 64: 48 7.3 / 7.3, 64 7.9 / 7.7, 96 8.9 / 8.2; 8 on 8 of 64: 96 10.1 / 10.2, 128 11.5 / 11.0
 // The host knows the longest history only, and shorter ones in the same caches gain from one launch
-// (16 on 8 of 128 at 260 positions of 4096: 6.4 / 7.5). Past PVC_MAX_ITEMS the workgroups, which stay
+// (16 on 8 of 128 at 260 positions of 4096: 6.7 / 7.4). Past PVC_MAX_ITEMS the workgroups, which stay
 // until their stores are acknowledged, no longer fit the device at once: 16 on 16 of 128, 64 blocks
-// 12.2 / 13.4, 96 16.5 / 15.8, 128 24.9 / 18.6.
+// 12.2 / 13.0, 96 16.2 / 15.6, 128 24.3 / 18.2.
 // ------------------------------------------------------------------------------------------
 
 constexpr int PVC_MAX_FLOATS = 32768;  // partials of a kv head: blocks of the longest history x REP * D
