@@ -1775,13 +1775,13 @@ struct Shape {
     static constexpr int SPLIT_BLOCKS = H <= 1024 ? 8 : H <= 2048 ? 7 : 9;
     // STEP_AUTO's switch to the hipGraph step (at most the kernel's longest history): the crossover of
     // the split instance's and the graph's time per token, measured on MI355X (us, 32 greedy tokens after
-    // an N(0, 1) cache; split / graph): 4B 4000 2038 / 2056, 4100 2076 / 2070, 4300 2132 / 2069, 5000
-    // 2237 / 2080, 8200 2250 / 2200, 10000 2385 / 2230; 1.7B 4250 1131 / 1160, 4416 1158 / 1166, 4500
-    // 1172 / 1160, 5000 1270 / 1153, 8300 1260 / 1246, 10000 1319 / 1263; 0.6B: the kernel at every length
-    // it holds (8200 774 / 947). From 64 blocks on a half-slot of the kernel runs a second item, while the
-    // graph's passes grow smoothly. The small test shape keeps a switch (736) so that a generate_greedy
-    // crossing it is exercised.
-    static constexpr int SWITCH_POS = H < 1024 ? 736 : H <= 1024 ? 1 << 30 : H <= 2048 ? 4480 : 4096;
+    // an N(0, 1) cache; split / graph): 4B 4000 2034 / 2059, 4100 2082 / 2100, 4300 2135 / 2103, 5000
+    // 2242 / 2112, 7000 2258 / 2194, 8200 2269 / 2265, 10000 2399 / 2294; 1.7B 4250 1158 / 1177, 4416
+    // 1194 / 1174, 5000 1227 / 1175, 6000 1260 / 1191, 8300 1278 / 1274, 10000 1361 / 1287; 0.6B: the
+    // kernel at every length it holds (8200 769 / 940). From 64 blocks on a half-slot of the kernel runs a
+    // second item, while the graph's passes grow smoothly. The small test shape keeps a switch (736) so
+    // that a generate_greedy crossing it is exercised.
+    static constexpr int SWITCH_POS = H < 1024 ? 736 : H <= 1024 ? 1 << 30 : H <= 2048 ? 4352 : 4224;
     // The split attention's statistics (block and global max and sum) reduce with their xor-4
     // and xor-8 steps through ds_swizzle (LDS8) where two query heads share a kv head, through
     // DPP at 4B (four): 0.6B after 8192 positions 1235-1237 tokens/s against 1185-1194 with DPP;

@@ -1004,7 +1004,7 @@ def test_persistent_step_wide_shapes_long_history(gpu, oracle, size):
         dec.close()
 
 
-@pytest.mark.parametrize("size,switch", [("1.7B", 4480), ("4B", 4096)])
+@pytest.mark.parametrize("size,switch", [("1.7B", 4352), ("4B", 4224)])
 def test_auto_step_switches_wide_shapes(gpu, oracle, size, switch):
     """STEP_AUTO's switch from the persistent kernel to the hipGraph at the 1.7B and 4B widths (2 layers,
     caches filled with N(0, 1)): single steps on both sides of it, with logits and argmax bit-identical
