@@ -473,7 +473,7 @@ def test_attention_position_outside_the_caches(gpu, fused, max_seq):
             gpu.attention_forward(out, x[0], cache[0], cache[1], att, hq, hkv, D, dev_i32([pos]), max_seq,
                                   0.1)
         torch.cuda.synchronize()
-        assert not out.any(), pos
+        assert not out.view(torch.int16).any(), pos  # +0 in every bit
         assert torch.equal(cache, held[0]) and torch.equal(att, held[1]), pos
 
 
