@@ -477,6 +477,31 @@ def test_attention_position_outside_the_caches(gpu, fused, max_seq):
         assert torch.equal(cache, held[0]) and torch.equal(att, held[1]), pos
 
 
+@pytest.mark.parametrize("hq,hkv,D,max_seq", [(2, 2, 64, 640), (16, 8, 128, 640), (8, 1, 256, 640),
+                                              (16, 8, 128, 9000)])
+def test_attention_scores_not_numbers(gpu, oracle, hq, hkv, D, max_seq):
+    """Scores that are NaN of every payload, or infinite, in all or the first blocks of a kv head (whose
+    first block's max also counts the head's items where PV and combine are one launch): every output is
+    written, NaN where the oracle's is and its bits elsewhere."""
+    import torch
+    ident(f"attention with scores that are not numbers {hq}/{hkv} D{D} of {max_seq}")
+    rng = np.random.default_rng(hq + D)
+    pos, scale = 600, float(np.float32(1.0 / np.sqrt(D)))
+    q, kc, vc = rand_bf16(rng, hq * D), rand_bf16(rng, (max_seq, hkv * D)), rand_bf16(rng, (max_seq, hkv * D))
+    att = torch.zeros(gpu.attention_workspace_floats(hq, D, max_seq), device="cuda")
+    for bits in (0xFFFF, 0x7FFF, 0x7F81, 0xFF81, 0x7FC0, 0x7F80, 0xFF80):
+        for rows in (slice(0, max_seq), slice(0, 64), slice(0, 1), slice(64, 128)):
+            keys = kc.copy()
+            keys[rows, :D] = bits  # the first kv head's
+            out = dev(np.full(hq * D, 0x1234, np.uint16))
+            gpu.attention_forward(out, dev(q), dev(keys), dev(vc), att, hq, hkv, D, dev_i32([pos]), max_seq,
+                                  scale)
+            want = oracle.attention(q, keys, vc, hq, hkv, D, pos, scale, oracle.GPU_ORDER)
+            got, nan = host(out), np.isnan(bf16_vals(want))
+            assert np.array_equal(got[~nan], want[~nan]), (hex(bits), rows)
+            assert np.isnan(bf16_vals(got)[nan]).all(), (hex(bits), rows)
+
+
 # the shapes whose last blocks' workgroups are the most and the largest
 @pytest.mark.parametrize("hq,hkv,D,max_seq", [(64, 8, 128, 2048), (64, 8, 256, 1024), (64, 8, 128, 8192),
                                               (32, 8, 256, 2048)])
