@@ -157,9 +157,9 @@ enum { ATTN_AUTO = 0, ATTN_SEPARATE = 1, ATTN_IN_SCORES = 2, ATTN_ONE_PASS = 3 }
  * per query head up to 448 / 384 / 512 positions at 0.6B / 1.7B / 4B, and split over
  * (kv head, 64-position block) items on every workgroup from there on. The switch is the kernel's
  * longest history at 0.6B (12288 positions on 256 CUs), 4352 positions at 1.7B and 4224 at 4B, from
- * where the graph leads by 0.2-6%. 5-token prompt, 256 tokens: 2523 / 1153 / 617 tokens/s
- * (the graph over 32 tokens: 1381 / 951 / 519); 0.6B after 4096 / 8192 positions 1520 / 1288 against
- * 1228 / 1109. Other shapes: the hipGraph. STEP_GRAPH: always the hipGraph. STEP_PERSISTENT: the
+ * where the graph leads by 0.2-6%. 5-token prompt, 256 tokens: 2493-2553 / 1155 / 618
+ * tokens/s (the graph over 32 tokens: 1399 / 962 / 529); 0.6B after 4096 / 8192 positions 1543 / 1283
+ * against 1193 / 1065. Other shapes: the hipGraph. STEP_GRAPH: always the hipGraph. STEP_PERSISTENT: the
  * persistent kernel at every position (max_seq at most the kernel's longest history) or an
  * error. */
 enum { STEP_AUTO = 0, STEP_GRAPH = 1, STEP_PERSISTENT = 2 };

@@ -118,8 +118,7 @@ void rmsnorm_gate_up_forward(bf16 *act, const bf16 *w_gate, const bf16 *w_up, co
                              hipStream_t stream);
 
 /* No counterpart in the reference: qk_norm_rope_forward followed by attention_forward
- * (src/kernels.cuh:18-24) for one decode position, with the same bits, in three launches
- * instead of four: the per-head QK-norm + RoPE is computed inside the attention's scores pass,
+ * (src/kernels.cuh:18-24) for one decode position, with the same bits, in one launch fewer: the per-head QK-norm + RoPE is computed inside the attention's scores pass,
  * per block of positions, while the block's keys stream. q and k are read, not rewritten; k'
  * and v are written to the caches' row *d_pos as qk_norm_rope_forward writes them. `att`, the
  * shapes, alignment and positions outside the caches are attention_forward's. */

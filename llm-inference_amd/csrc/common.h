@@ -352,10 +352,10 @@ __device__ __forceinline__ void wave_amax(float &v, int &i) {
 //
 // Outside [-105, 90] the argument is clamped, which gives 0 (e^-104 is already below half the smallest
 // denormal) and inf (e^89 is past the largest float) as the limits do; NaN is put back at the end. The
-// same bits as the form with early returns (BRANCHES), for every fp32 input (checked on the GPU). That
+// same bits as the form with early returns (BRANCHES), for every fp32 input (a GPU test compares them). That
 // form has up to four branches around each call, so the exponentials of a wave run one after the other:
-// attention at Qwen3-0.6B's widths and 260 positions 15.25 -> 14.86 us without them, the step kernel
-// with one workgroup per head 400.9 -> 398.3 us per token. The step kernel's split instance keeps them
+// attention at Qwen3-0.6B's widths and 260 positions 15.25 -> 14.86 us without them; the step kernel with
+// one workgroup per head measures the same within its runs' noise. The step kernel's split instance keeps them
 // where they measured faster (its SiLU, and at 4B its attention, where they hold an item's statistics
 // and their stores together, ahead of the next item's).
 template <bool BRANCHES = false>

@@ -1952,8 +1952,8 @@ int step_kernel_split_blocks(const Config *cfg) {
     return 0;
 }
 
-// Measured on MI355X, 32 tokens from position 5: 0.6B 373 us per token (step kernel) against 724
-// (hipGraph), 1.7B 874 against 1051, 4B 1603 against 1925.
+// Measured on MI355X, 32 tokens from position 5: 0.6B 377 us per token (step kernel) against 715
+// (hipGraph), 1.7B 874 against 1039, 4B 1600 against 1890.
 int step_kernel_switch_pos(const Config *cfg) {
     int sw = 0;
 #define SWITCH(S)                                                                           \

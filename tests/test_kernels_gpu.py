@@ -384,14 +384,14 @@ def test_attention_head_dims(gpu, oracle, D, rep):
                                              oracle.EXACT)).max() <= 2
 
 
-# combine widths: one item per kv head (nb = 1), every column count down to 16, the cap on waiting
-# items (REP 8 of 256), two staged chunks of partials, and more items than one launch takes (8200)
+# one item per kv head (nb = 1), PV and combine in one launch and in two, more than one staged chunk of
+# partials (17000), and more items than a launch has workgroups (8200)
 @pytest.mark.parametrize("hq,hkv,D,pos,max_seq", [
     (2, 2, 64, 5, 64), (16, 2, 64, 700, 704), (4, 4, 256, 127, 128), (8, 8, 64, 17000, 17001),
     (64, 8, 256, 8200, 8256), (8, 1, 128, 9000, 9001), (8, 8, 64, 1000, 65600), (4, 4, 128, -1, 200)])
 def test_attention_one_launch_combine(gpu, oracle, hq, hkv, D, pos, max_seq):
-    """The PV pass and the combine in one launch: bit-identical to the oracle whatever `att` held
-    before (the mark of an unwritten partial, another call's partials), at a later and an earlier
+    """The PV pass and the combine: bit-identical to the oracle whatever `att` held
+    before (every bit set, another call's partials), at a later and an earlier
     position on the same workspace, and with NaN among the values. Position -1 (no history) gives
     zeros."""
     import torch

@@ -548,13 +548,11 @@ def test_graph_step_other_head_dims(gpu, oracle, head_dim, attn):
 
 @pytest.mark.parametrize("n_heads", [4, 8, 16, 32])
 def test_graph_step_pv_combine_one_launch(gpu, oracle, n_heads):
-    """At head_dim 128 the graph step runs attention's PV and combine passes as one launch
-    (attn_pv_combine_kernel): every item publishes its block partials as tagged words and the
-    items of the T last blocks of each kv head add them in block order, T the largest power of
-    two <= min(blocks, REP * 128 / 16). 4 kv heads with n_heads / 4 = 1, 2, 4 or 8 query heads
-    each, a 16580-position N(0, 1) cache: logits bit-identical to the oracle at positions holding
-    1 to 260 blocks (T = 1 to 32; two staged chunks of partials past 256 blocks), in both
-    attention forms, then a short generate_greedy equal to the oracle's."""
+    """The graph step's attention over a long cache, where PV and combine are two launches (one launch
+    for short caches: test_graph_step_pv_combine_small_grids). 4 kv heads with n_heads / 4 = 1, 2, 4 or
+    8 query heads each, a 16580-position N(0, 1) cache: logits bit-identical to the oracle at positions
+    holding 1 to 260 blocks (two staged chunks of partials past 256 blocks), in both attention forms,
+    then a short generate_greedy equal to the oracle's."""
     ident(f"graph step one-launch PV + combine, {n_heads}/4 heads")
     from llm_inference_amd import model
     max_seq = 16640
@@ -597,7 +595,7 @@ def test_graph_step_pv_combine_one_launch(gpu, oracle, n_heads):
 @pytest.mark.parametrize("n_heads,n_kv_heads,max_seq", [(8, 1, 100), (8, 8, 130), (2, 2, 64)])
 def test_graph_step_pv_combine_small_grids(gpu, oracle, n_heads, n_kv_heads, max_seq):
     """The one-launch PV + combine on small grids: one kv head with 8 query heads (1024 columns,
-    4 per thread when one item combines them all), 8 kv heads of one query head, and a cache of
+    4 per thread in the combine), 8 kv heads of one query head, and a cache of
     a single 64-position block (one item per kv head, which both computes and combines). Every
     position of the cache stepped through in both attention forms: logits bit-identical to the
     oracle."""
@@ -1049,10 +1047,9 @@ def test_auto_step_switches_wide_shapes(gpu, oracle, size, switch):
 def test_step_keeps_an_earlier_error_code(gpu, mode):
     """A wait between workgroups that finds the error flag already set stops at once and leaves
     the code alone: with the flag set to 1 (token or position out of range) from the host before
-    a step whose attention waits on other workgroups (graph step: the PV + combine launch at
-    position 200, four blocks; persistent step: every tagged-vector poll), the error reported
-    afterwards is the out-of-range one, not a timed-out wait. Every wait ends at once, so the
-    kernels exit normally."""
+    a step (persistent: every tagged-vector poll waits on other workgroups; graph: nothing does), the
+    error reported afterwards is the out-of-range one, not a timed-out wait. Every wait ends at once,
+    so the kernels exit normally."""
     ident(f"earlier error code kept ({mode} step)")
     from llm_inference_amd import LlmError, model
     cfg = model.make_config(hidden_size=512, intermediate_size=1024, n_layers=2, n_heads=8,
