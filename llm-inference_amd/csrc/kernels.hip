@@ -2687,7 +2687,6 @@ __global__ __launch_bounds__(SAMPLE_T) void sample_kernel(int *out, const bf16 *
                                         __HIP_MEMORY_SCOPE_AGENT) == 0;
         if (s_taken)
             __hip_atomic_store(gptr(&sl.done), 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // before any work is open
     }
     float m = -__builtin_huge_valf();
     int done = 0;
@@ -2709,6 +2708,7 @@ __global__ __launch_bounds__(SAMPLE_T) void sample_kernel(int *out, const bf16 *
     for (int i = done + t; i < n; i += SAMPLE_T) m = fmaxf(m, bf2f(x[i]));
     m = wave_max(m);
     if ((t & 63) == 0) wmax[t >> 6] = m;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the slot's count is zero before any work is open
     __syncthreads();
     float mx = wmax[0];
 #pragma unroll
